@@ -12,6 +12,9 @@
 // with a fixed order, so results are deterministic and no floating-point atomics are used.  Every
 // CSR value and rhs entry is written exactly once, the values with coalesced stores.
 //
+// The specialised simplices take another route to the same row-owner sums, by block lists (assemble_lists_wg);
+// the staged reduction above serves the generic expression, and specialised systems whose plan does not fit.
+//
 // Element mathematics (reference files relative to the coolfluid3 tree):
 //   specialised P1 triangle / tetrahedron: plugins/UFEM/src/UFEM/NavierStokesSpecializations.hpp:38-303
 //     (incl. the vk for wk substitution of lines 224-226 and 236-238 and tau from the velocity u)
@@ -46,7 +49,9 @@ struct SpecP1 {
   R ua[D];          // mean advection velocity u_avg
   R na[D];          // normal of the row node a
   R Q[D];           // velocity-row coefficient: skew-symmetric advection + stress diffusion + bulk
-  R cc, nudV, cpres, tpdV, pn, pp, tdo, tdd, tpc;
+  R tsdV, nudV, visc, m0dt;   // element: tau / (D^2 V), nu / (D^2 V), nu / (3 D^2 V) + tau_bulk / (D^2 V), V / (12|20 dt)
+  R tsu;
+  R cc, cpres, pn, pp, tdo, tdd, tpc;
   int a;
 
   // geometry in type T: normals and volume
@@ -100,23 +105,31 @@ struct SpecP1 {
         gsq += (i == l ? T(1) : T(2)) * gil * gil;
         if(i == l) tr += gil;
       }
-    const T sq = sqrt(f4dt2 + adv + T(16) * (nu * nu * gsq));
-    t_su = T(1) / sq;
-    t_bu = sq / tr;
+    const T q = f4dt2 + adv + T(16) * (nu * nu * gsq);
+    t_su = inv_sqrt(q);
+    t_bu = (q * t_su) * reciprocal(tr);
   }
 
   __device__ __forceinline__ void prepare(const AsmArgs& g, uint32_t e, int a_)
   {
     load_conn<K>(g.conn, e, cn);
-    prepare_nodes(g, g.xp, g.st, g.ad, a_);
+    prepare_element(g, [&](uint32_t nd, double* x, double* u, double* w, double& nu) {
+      double xp[4], st[4], ad[4];
+      unpack(g.xp[nd], xp);
+      unpack(g.st[nd], st);
+      unpack(g.ad[nd], ad);
+#pragma unroll
+      for(int d = 0; d < D; ++d) { x[d] = xp[d]; u[d] = st[d]; w[d] = ad[d]; }
+      nu = ad[3];
+    });
+    prepare_row(g, a_);
   }
 
-  // element quantities from the packed node records xp/st/ad (global, or the workgroup's LDS copy),
-  // cn[] indexing them
-  __device__ __forceinline__ void prepare_nodes(const AsmArgs& g, const double4* xpr, const double4* str,
-                                                const double4* adr, int a_)
+  // element quantities from the coordinates, velocity, advection velocity and viscosity that node(cn[m], ...)
+  // gives
+  template<class Node>
+  __device__ __forceinline__ void prepare_element(const AsmArgs& g, Node node)
   {
-    a = a_;
     double X[K][D];
     double uc[D];
     double nus = 0.;
@@ -124,17 +137,14 @@ struct SpecP1 {
     for(int d = 0; d < D; ++d) { uc[d] = 0.; uas[d] = R(0); }
 #pragma unroll
     for(int m = 0; m < K; ++m) {
-      double xp[4], st[4], ad[4];
-      unpack(xpr[cn[m]], xp);
-      unpack(str[cn[m]], st);
-      unpack(adr[cn[m]], ad);
+      double u[D], w[D], nun;
+      node(cn[m], X[m], u, w, nun);
 #pragma unroll
       for(int d = 0; d < D; ++d) {
-        X[m][d] = xp[d];
-        uc[d] += st[d];
-        uas[d] += (R)ad[d];
+        uc[d] += u[d];
+        uas[d] += (R)w[d];
       }
-      nus += ad[3];
+      nus += nun;
     }
     for(int d = 0; d < D; ++d) {
       uc[d] = uc[d] * (1.0 / K);
@@ -142,7 +152,7 @@ struct SpecP1 {
     }
     const double nu_mean = fabs(nus * (1.0 / K));
     const R nu = (R)nu_mean;
-    R V = R(0), invV, tsu, tbu;
+    R V = R(0), invV, tbu;
     bool fp64_geom = sizeof(R) == sizeof(double);
     if constexpr(sizeof(R) != sizeof(double)) {
       // coordinates relative to node 0, formed in FP64: the FP32 differences of absolute coordinates
@@ -167,7 +177,7 @@ struct SpecP1 {
     if(fp64_geom) {
       double n64[K][D], V64, ts, tb;
       geometry<double>(X, n64, V64);
-      const double iv = 1. / V64;
+      const double iv = reciprocal(V64);
       tau_metric<double>(n64, iv * (1.0 / D), uc, nu_mean, g.f4dt2, ts, tb);
       for(int m = 0; m < K; ++m)
         for(int d = 0; d < D; ++d) n[m][d] = (R)n64[m][d];
@@ -178,15 +188,26 @@ struct SpecP1 {
         // det J of the Jacobian, as the reference's ComputeTau does (SUPG.hpp:178, ElementData.hpp:302-314)
         const double Vr = tet_volume_ref(X);
         V = Vr;
-        invV = 1. / Vr;
+        invV = reciprocal(Vr);
       }
     } else {
       R ucr[D];
       for(int d = 0; d < D; ++d) ucr[d] = (R)uc[d];
-      invV = R(1) / V;
+      invV = reciprocal(V);
       tau_metric<R>(n, invV * R(1.0 / D), ucr, nu, (R)g.f4dt2, tsu, tbu);
       if(!(V > R(0))) g.status[0] = 1;
     }
+    const R rdV = invV * R(1.0 / (D * D));
+    tsdV = tsu * rdV;
+    nudV = nu * rdV;
+    visc = nudV * R(1.0 / 3.0) + tbu * rdV;
+    m0dt = (R)g.invdt * (V * R(D == 2 ? 1.0 / 12.0 : 1.0 / 20.0));
+  }
+
+  // coefficients of the row of local node a_
+  __device__ __forceinline__ void prepare_row(const AsmArgs& g, int a_)
+  {
+    a = a_;
     // normal of the row node, selected without dynamic register indexing
 #pragma unroll
     for(int d = 0; d < D; ++d) na[d] = n[0][d];
@@ -197,10 +218,6 @@ struct SpecP1 {
         for(int d = 0; d < D; ++d) na[d] = n[m][d];
     // per-row (node a) coefficients (NavierStokesSpecializations.hpp:66-145 / 196-301)
     const R c0 = R(D == 2 ? 1.0 / 6.0 : 1.0 / 12.0);
-    const R rdV = invV * R(1.0 / (D * D));
-    const R tsdV = tsu * rdV;
-    nudV = nu * rdV;
-    const R tbdV = tbu * rdV;
     R u_ni = R(0);
     for(int d = 0; d < D; ++d) u_ni += ua[d] * na[d];
     const R cskew = R(0.5) * c0 + R(0.5) * tsdV * u_ni;
@@ -211,19 +228,16 @@ struct SpecP1 {
     // n_i . u~ with the tetrahedron substitution of vk for wk (lines 236-238)
     R ni_ut = na[0] * ua[0] + na[1] * ua[1];
     if constexpr(D == 3) ni_ut += na[2] * ua[1];
-    const R visc = nudV * R(1.0 / 3.0) + tbdV;
 #pragma unroll
     for(int r = 0; r < D; ++r) {
       const R uk = ua[(D == 3 && r == 2) ? 1 : r];   // W rows use vk (lines 224-226)
       Q[r] = cskew * uk + visc * na[r];
     }
-    tpdV = tsdV;   // tau_ps = tau_su
-    pn = R(0.5) * tpdV * ni_ut + c0;
-    pp = tpdV * inv_rho;
-    const R m0 = V * R(D == 2 ? 1.0 / 12.0 : 1.0 / 20.0);
+    pn = R(0.5) * tsdV * ni_ut + c0;   // tau_ps = tau_su
+    pp = tsdV * inv_rho;
     const R invdt = (R)g.invdt;
-    tdo = invdt * (m0 + time_ii);
-    tdd = invdt * (R(2) * m0 + time_ii);
+    tdo = m0dt + invdt * time_ii;
+    tdd = tdo + m0dt;
     tpc = invdt * tsu * c0;
   }
 
@@ -257,7 +271,7 @@ struct SpecP1 {
     {
       R Ar[NEQ];
 #pragma unroll
-      for(int c = 0; c < D; ++c) Ar[c] = uknj * (tpdV * na[c]) + pn * nj[c];
+      for(int c = 0; c < D; ++c) Ar[c] = uknj * (tsdV * na[c]) + pn * nj[c];
       Ar[D] = pp * ninj;
       if constexpr(RHS) {
         R s = R(0);
@@ -574,11 +588,7 @@ struct GenericP1 {
 // right-hand side, which is formed by the FP64 pass.
 // ---------------------------------------------------------------------------------------------
 // the work of one assembly workgroup (row range wg of the system described by g)
-// STAGED (specialised simplices with node staging): the workgroup's range bounds come from one
-// 32-byte header, the records of its distinct nodes are copied into LDS once, and every element
-// gather and nodal state read of the passes is an LDS read (three dependent global loads per
-// workgroup instead of five, and one global read per distinct node instead of one per incidence).
-template<class Op, typename R, typename VR, bool RHS, bool STAGED = false>
+template<class Op, typename R, typename VR, bool RHS>
 __device__ __forceinline__ void assemble_wg(const AsmArgs& g, uint32_t wg)
 {
   constexpr int K = Op::K, NEQ = Op::NEQ, NN = NEQ * NEQ;
@@ -592,28 +602,11 @@ __device__ __forceinline__ void assemble_wg(const AsmArgs& g, uint32_t wg)
   __shared__ uint32_t s_rowinc[kThreads + 1];
   __shared__ uint16_t s_acc[kThreads];
 
-  uint32_t r0, r1, i0, ninc, blk0, nblk, n0 = 0, nn = 0;
-  if constexpr(STAGED) {
-    const uint4 h0 = reinterpret_cast<const uint4*>(g.wg_head)[2 * wg];
-    const uint4 h1 = reinterpret_cast<const uint4*>(g.wg_head)[2 * wg + 1];
-    r0 = h0.x; r1 = h0.y; i0 = h0.z; ninc = h0.w - h0.z;
-    blk0 = h1.x; nblk = h1.y - h1.x; n0 = h1.z; nn = h1.w - h1.z;
-  } else {
-    r0 = g.wg_rows[wg]; r1 = g.wg_rows[wg + 1];
-    i0 = g.inc_ptr[r0]; ninc = g.inc_ptr[r1] - i0;
-    blk0 = g.row_ptr[r0]; nblk = g.row_ptr[r1] - blk0;
-  }
+  const uint32_t r0 = g.wg_rows[wg], r1 = g.wg_rows[wg + 1];
+  const uint32_t i0 = g.inc_ptr[r0], ninc = g.inc_ptr[r1] - i0;
+  const uint32_t blk0 = g.row_ptr[r0], nblk = g.row_ptr[r1] - blk0;
   const uint32_t nrows = r1 - r0;
   const int t = threadIdx.x;
-  // node staging area (dynamic LDS): xp records [0, nn), st [nn, 2 nn), ad [2 nn, 3 nn)
-  extern __shared__ double4 s_nodes[];
-  if constexpr(STAGED)
-    for(uint32_t j = t; j < nn; j += kThreads) {
-      const uint32_t nd = g.wg_nodes[n0 + j];
-      s_nodes[j] = g.xp[nd];
-      s_nodes[nn + j] = g.st[nd];
-      s_nodes[2 * nn + j] = g.ad[nd];
-    }
   if constexpr(RHS)
     for(uint32_t j = t; j <= nrows; j += kThreads) s_rowinc[j] = g.inc_ptr[r0 + j] - i0;
   if((uint32_t)t < nblk) s_acc[t] = g.blk_acc[blk0 + t];
@@ -624,27 +617,12 @@ __device__ __forceinline__ void assemble_wg(const AsmArgs& g, uint32_t wg)
   R rhs[NEQ];
 #pragma unroll
   for(int r = 0; r < NEQ; ++r) rhs[r] = R(0);
-  if constexpr(STAGED) {
-    uint32_t ea = 0, loc = 0;
-    if(active) {
-      posw = reinterpret_cast<const uint32_t*>(g.inc_pos)[i0 + t];
-      ea = g.inc[i0 + t];
-      loc = g.inc_loc[i0 + t];
-    }
-    __syncthreads();   // node records staged
-    if(active) {
-#pragma unroll
-      for(int m = 0; m < K; ++m) op.cn[m] = (loc >> (8 * m)) & 255u;
-      op.prepare_nodes(g, s_nodes, s_nodes + nn, s_nodes + 2 * nn, (int)(ea % K));
-    }
-  } else {
-    if(active) {
-      posw = reinterpret_cast<const uint32_t*>(g.inc_pos)[i0 + t];
-      const uint32_t ea = g.inc[i0 + t];
-      op.prepare(g, ea / K, (int)(ea % K));
-    }
-    __syncthreads();
+  if(active) {
+    posw = reinterpret_cast<const uint32_t*>(g.inc_pos)[i0 + t];
+    const uint32_t ea = g.inc[i0 + t];
+    op.prepare(g, ea / K, (int)(ea % K));
   }
+  __syncthreads();
   // accumulator thread t: block bs of this workgroup, rank h of c; rows [beg_p + h, end_p) step c
   const uint32_t alast = s_acc[nblk - 1];
   const uint32_t n_acc = (alast & 255u) + (alast >> 8);
@@ -670,7 +648,7 @@ __device__ __forceinline__ void assemble_wg(const AsmArgs& g, uint32_t wg)
     constexpr int B = decltype(bc)::value;
     if(active) {
       R xb[NEQ];
-      if constexpr(RHS) load_state<NEQ, R>(STAGED ? s_nodes + nn : g.st, op.cn[B], xb);
+      if constexpr(RHS) load_state<NEQ, R>(g, op.cn[B], xb);
       op.template block<B, RHS, VR>(g, s_blk + ((posw >> (8 * B)) & 255u) * LDW, rhs, xb);
     }
     __syncthreads();
@@ -730,10 +708,289 @@ __device__ __forceinline__ void assemble_wg(const AsmArgs& g, uint32_t wg)
 }
 
 // FP32 kernels: at most 96 VGPRs, so that 5 waves fit per SIMD (104 would allow 4)
-template<class Op, typename R, typename VR, bool RHS, bool STAGED>
+template<class Op, typename R, typename VR, bool RHS>
 __global__ __launch_bounds__(kThreads, sizeof(R) == sizeof(float) ? 5 : 1) void k_assemble(AsmArgs g)
 {
-  assemble_wg<Op, R, VR, RHS, STAGED>(g, xcd_order(blockIdx.x, gridDim.x));
+  assemble_wg<Op, R, VR, RHS>(g, xcd_order(blockIdx.x, gridDim.x));
+}
+
+// ---------------------------------------------------------------------------------------------
+// Specialised simplices by block lists: the work of one plan (sparsity.hip)
+//   1. one element per thread: face normals, n . u_avg and six scalars, written to LDS as its record;
+//   2. one thread per block list (a CSR block, or plan_list_length of its contributions): the operator sums
+//      A and T of the block straight from the records, in registers;
+//   3. combine (M = T / dt + theta A) once per list, with its share of the rhs, -A x_b; the lists of a block
+//      are added in order through LDS and stored in the order of the values.
+// The staged reduction (assemble_wg) instead computes an element once per owned row, forms every element
+// block of 16 values, writes it to LDS and reads it back, K passes with two barriers each, and repeats the
+// combine and the rhs product for every one.
+// Measured (kernel, us, staged reduction -> block lists): FP64 tetrahedra 61^3 cells 389 -> 264, 128^3
+// 3147 -> 2179; FP32 208 -> 143, 1811 -> 1139; triangles 700^2 140 -> 120 (FP64), 81 -> 68 (FP32).
+// At 61^3: 1160 -> 990 VALU instructions per wave and 5/6 of the waves, 25 % fewer LDS instructions; VALU and LDS are each
+// busy about 60 % of the time with 5 to 6 workgroups per CU, and neither HBM (1.9 TB/s) nor the load chain at
+// the start bounds it: a persistent form that loads the next plan and its nodes during the block sums was no
+// faster (its 159 VGPRs cost the waves that hid the same latency).
+// dynamic LDS: [nodal states] [other nodal data; then the element records; then the block rows and rhs
+// parts], the states kept to the end with RHS.  The nodal data are arrays of 16-byte pairs, (u, v), (w, p),
+// (x, y), (z, nu), (u_adv x, y), and u_adv z: whole 32-byte records would put every first half on the same
+// half of the banks.
+template<int D, typename R>
+struct PlanLayout {
+  static constexpr int K = D + 1, NEQ = D + 1, NN = NEQ * NEQ;
+  static constexpr int COL = D + 1;         // n_b, n_b . u_avg
+  static constexpr int ELEM = K * COL;      // tau/(D^2 V), nu/(D^2 V), viscous + bulk, u_avg x, y, V/(12|20 dt)
+  static constexpr int WORDS = ELEM + 6;
+  // record stride: an odd number of 16-byte pieces, so that the records spread over the banks
+  static constexpr int STRIDE = (((WORDS * (int)sizeof(R) + 15) / 16) | 1) * 16 / (int)sizeof(R);
+  static constexpr int LDW = D == 3 ? lds_row<R, NN>() : NN;   // 9 values: odd by themselves
+  static size_t lds_bytes(bool rhs, uint32_t nodes, uint32_t elems, uint32_t lists)
+  {
+    const size_t stage = (size_t)nodes * (rhs ? 56 : 88);
+    const size_t rec = sizeof(R) * STRIDE * (elems + 1);
+    const size_t row = sizeof(R) * (LDW + (rhs ? NEQ : 0)) * lists;
+    return (rhs ? sizeof(double4) * nodes : 0) + std::max(stage, std::max(rec, row));
+  }
+};
+
+template<int D, typename R, bool RHS>
+__device__ __forceinline__ void assemble_lists_wg(const AsmArgs& g, uint32_t wg, unsigned char* smem)
+{
+  typedef PlanLayout<D, R> Y;
+  constexpr int K = Y::K, NEQ = Y::NEQ, NN = Y::NN, LDW = Y::LDW;
+  constexpr int LEN = (int)plan_list_length(K);
+  __shared__ uint16_t s_first[kThreads + 1];                // first list of each block
+  __shared__ uint16_t s_rowfirst[RHS ? kThreads + 1 : 1];   // first list of each row
+  __shared__ uint32_t s_wave[2][kThreads / 64];
+
+  const uint32_t t = threadIdx.x, ns = g.plan_nodes;
+  const unsigned char* plan = g.plan + (uint64_t)wg * plan_bytes(ns);
+  const uint32_t* nodes = reinterpret_cast<const uint32_t*>(plan + kPlanHeadBytes);
+  const uint32_t* locs = nodes + ns;
+  const uint64_t* los = reinterpret_cast<const uint64_t*>(locs + kThreads);
+  const uint32_t loc = locs[t];
+  const uint64_t lo = los[t];
+  const uint32_t hi = reinterpret_cast<const uint16_t*>(los + kThreads)[t];
+  double2* s_uv = reinterpret_cast<double2*>(smem);
+  double2* s_wp = s_uv + ns;
+  unsigned char* body = smem + (RHS ? 2 * sizeof(double2) * ns : 0);
+  double2* s_xy = RHS ? reinterpret_cast<double2*>(body) : s_wp + ns;
+  double2* s_zn = s_xy + ns;
+  double2* s_ad = s_zn + ns;
+  double* s_az = reinterpret_cast<double*>(s_ad + ns);
+  R* s_rec = reinterpret_cast<R*>(body);
+  R* s_row = reinterpret_cast<R*>(body);
+  R* s_rhs = s_row + LDW * g.plan_lists;
+  for(uint32_t j = t; j < ns; j += kThreads) {
+    const uint32_t nd = nodes[j];
+    const double4 xp = g.xp[nd], st = g.st[nd], ad = g.ad[nd];
+    s_xy[j] = make_double2(xp.x, xp.y);
+    s_zn[j] = make_double2(xp.z, ad.w);
+    s_uv[j] = make_double2(st.x, st.y);
+    s_wp[j] = make_double2(st.z, st.w);
+    s_ad[j] = make_double2(ad.x, ad.y);
+    if constexpr(D == 3) s_az[j] = ad.z;
+  }
+  const uint4 h0 = reinterpret_cast<const uint4*>(plan)[0], h1 = reinterpret_cast<const uint4*>(plan)[1];
+  const uint32_t r0 = h0.x, nrows = h0.y, ne = h0.z, blk0 = h1.x, nblk = h1.y, nlists = h1.z;
+  __syncthreads();
+  SpecP1<D, R> op;
+  if(t < ne) {
+#pragma unroll
+    for(int m = 0; m < K; ++m) op.cn[m] = (loc >> (8 * m)) & 255u;
+    op.prepare_element(g, [&](uint32_t nd, double* x, double* u, double* w, double& nu) {
+      const double2 xy = s_xy[nd], zn = s_zn[nd], uv = s_uv[nd], ad = s_ad[nd];
+      x[0] = xy.x; x[1] = xy.y;
+      u[0] = uv.x; u[1] = uv.y;
+      w[0] = ad.x; w[1] = ad.y;
+      if constexpr(D == 3) { x[2] = zn.x; u[2] = s_wp[nd].x; w[2] = s_az[nd]; }
+      nu = zn.y;
+    });
+  }
+  const uint64_t bstart = __ballot(lo >> 63), rstart = __ballot(hi >> 15);
+  if((t & 63u) == 0) {
+    s_wave[0][t >> 6] = (uint32_t)__popcll(bstart);
+    s_wave[1][t >> 6] = (uint32_t)__popcll(rstart);
+  }
+  __syncthreads();   // the element records replace the node records
+  if(t < ne) {
+    R* rec = s_rec + t * Y::STRIDE;
+#pragma unroll
+    for(int b = 0; b < K; ++b) {
+      R un = R(0);
+#pragma unroll
+      for(int d = 0; d < D; ++d) {
+        rec[b * Y::COL + d] = op.n[b][d];
+        un += op.ua[d] * op.n[b][d];
+      }
+      rec[b * Y::COL + D] = un;
+    }
+    rec[Y::ELEM] = op.tsdV;
+    rec[Y::ELEM + 1] = op.nudV;
+    rec[Y::ELEM + 2] = op.visc;
+    rec[Y::ELEM + 3] = op.ua[0];
+    rec[Y::ELEM + 4] = op.ua[1];
+    rec[Y::ELEM + 5] = op.m0dt;
+  }
+  if(t < (uint32_t)Y::WORDS) s_rec[ne * Y::STRIDE + t] = R(0);   // the record of the unused list entries
+  // block of this thread's list; row of the LDS rows: the first list of a block at its block, the others
+  // behind the blocks in order
+  uint32_t blk = (uint32_t)__popcll(bstart & (~0ull >> (63 - (t & 63u)))) - 1;
+  for(uint32_t v = 0; v < (t >> 6); ++v) blk += s_wave[0][v];
+  const uint32_t lds_row_t = (lo >> 63) ? blk : nblk + (t - blk - 1);
+  if(lo >> 63) s_first[blk] = (uint16_t)t;
+  if(RHS && (hi >> 15)) {
+    uint32_t row = (uint32_t)__popcll(rstart & ((1ull << (t & 63u)) - 1));
+    for(uint32_t v = 0; v < (t >> 6); ++v) row += s_wave[1][v];
+    s_rowfirst[row] = (uint16_t)t;
+  }
+  if(t == 0) {
+    s_first[nblk] = (uint16_t)nlists;
+    if constexpr(RHS) s_rowfirst[nrows] = (uint16_t)nlists;
+  }
+  __syncthreads();
+
+  R A[D][D], up[D], pu[D], tp[D], S = R(0), pp = R(0), tu = R(0);
+#pragma unroll
+  for(int r = 0; r < D; ++r) {
+    up[r] = pu[r] = tp[r] = R(0);
+#pragma unroll
+    for(int c = 0; c < D; ++c) A[r][c] = R(0);
+  }
+  if(t < nlists) {
+    // NavierStokesSpecializations.hpp:66-145 / 196-301, per contribution (element, row node a, column node b)
+    const R c0 = R(D == 2 ? 1.0 / 6.0 : 1.0 / 12.0);
+    const R ctp = R(D == 2 ? 8.0 : 15.0);   // c0 tau / dt = ctp (tau / (D^2 V)) (V / (12|20 dt))
+#pragma unroll
+    for(int i = 0; i < LEN; ++i) {
+      const uint32_t entry = i < 5 ? (uint32_t)(lo >> (11 * i)) & 2047u : hi & 2047u;
+      const R* rec = s_rec + (entry >> 4) * Y::STRIDE;
+      const R* ra = rec + ((entry >> 2) & 3u) * Y::COL;
+      const R* rb = rec + (entry & 3u) * Y::COL;
+      const bool diag = ((entry >> 2) & 3u) == (entry & 3u);
+      R na[D], nb[D], nanb = R(0);
+#pragma unroll
+      for(int d = 0; d < D; ++d) { na[d] = ra[d]; nb[d] = rb[d]; }
+      const R una = ra[D], unb = rb[D];
+      const R tsdV = rec[Y::ELEM], nudV = rec[Y::ELEM + 1], visc = rec[Y::ELEM + 2];
+      const R u0 = rec[Y::ELEM + 3], u1 = rec[Y::ELEM + 4], m0dt = rec[Y::ELEM + 5];
+#pragma unroll
+      for(int d = 0; d < D; ++d) nanb += na[d] * nb[d];
+      const R cc = c0 + tsdV * una;         // convection, standard and SUPG
+      const R hc = R(0.5) * cc, h0u = hc * u0, h1u = hc * u1;
+      // n_a . u~ with the tetrahedron substitution of vk for wk (lines 236-238)
+      R naut = na[0] * u0 + (D == 3 ? na[1] + na[D - 1] : na[1]) * u1;
+      const R pn = c0 + (R(0.5) * tsdV) * naut;
+      const R tpc = ctp * tsdV * m0dt;
+      const R tuo = m0dt + tpc * una;
+      S += cc * unb;
+      S += nudV * nanb;
+      pp += tsdV * nanb;                    // tau_ps = tau_su
+      tu += diag ? tuo + m0dt : tuo;
+      const R pua = tsdV * unb;
+#pragma unroll
+      for(int r = 0; r < D; ++r) {
+        const R Q = (r == 0 ? h0u : h1u) + visc * na[r];   // W rows use vk (lines 224-226)
+#pragma unroll
+        for(int c = 0; c < D; ++c) A[r][c] += Q * nb[c];
+        up[r] += cc * nb[r];
+        pu[r] += pua * na[r];
+        pu[r] += pn * nb[r];
+        tp[r] += tpc * na[r];
+      }
+    }
+  }
+  __syncthreads();   // the block rows replace the records
+  if(t < nlists) {
+    const R th = (R)g.theta, thq = (R)g.thq, inv_rho = (R)g.inv_rho;
+#pragma unroll
+    for(int r = 0; r < D; ++r) {
+      A[r][r] += S;
+      up[r] *= inv_rho;
+    }
+    pp *= inv_rho;
+    if constexpr(RHS) {
+      const uint32_t nd = (uint32_t)(lo >> 55) & 255u;
+      const double2 uv = s_uv[nd], wp = s_wp[nd];
+      const double st[4] = {uv.x, uv.y, wp.x, wp.y};
+      R xb[NEQ];
+#pragma unroll
+      for(int c = 0; c < NEQ; ++c) xb[c] = (R)st[c];
+#pragma unroll
+      for(int r = 0; r < D; ++r) {
+        R s = up[r] * xb[D];
+#pragma unroll
+        for(int c = 0; c < D; ++c) s += A[r][c] * xb[c];
+        s_rhs[t * NEQ + r] = s;
+      }
+      R s = pp * xb[D];
+#pragma unroll
+      for(int c = 0; c < D; ++c) s += pu[c] * xb[c];
+      s_rhs[t * NEQ + D] = s;
+    }
+    R m[NN];
+#pragma unroll
+    for(int r = 0; r < D; ++r) {
+#pragma unroll
+      for(int c = 0; c < D; ++c) m[r * NEQ + c] = th * A[r][c] + (r == c ? tu : R(0));
+      m[r * NEQ + D] = th * up[r];
+      m[D * NEQ + r] = tp[r] + thq * pu[r];
+    }
+    m[NN - 1] = thq * pp;
+#pragma unroll
+    for(int q = 0; q < NN; ++q) s_row[lds_row_t * LDW + q] = m[q];
+  }
+  __syncthreads();
+  {
+    // 16 bytes per lane where a block is a multiple of that (D = 3)
+    constexpr int W = (NN * sizeof(R)) % 16 == 0 ? 16 / sizeof(R) : 1;
+    constexpr int P = NN / W;   // pieces per block
+    struct alignas(W * sizeof(R)) Piece { R v[W]; };
+    Piece* dst = reinterpret_cast<Piece*>(static_cast<R*>(g.values) + (uint64_t)blk0 * NN);
+    constexpr int U = 4;        // pieces in flight per thread
+    for(uint32_t o = t; o < nblk * P; o += U * kThreads) {
+      Piece sum[U];
+      uint32_t f[U], l[U];
+#pragma unroll
+      for(int u = 0; u < U; ++u) {
+        const uint32_t ou = min(o + u * kThreads, nblk * P - 1), sb = ou / P;
+        sum[u] = *reinterpret_cast<const Piece*>(s_row + sb * LDW + (ou % P) * W);
+        f[u] = s_first[sb];
+        l[u] = s_first[sb + 1];
+      }
+#pragma unroll
+      for(int u = 0; u < U; ++u) {
+        const uint32_t ou = o + u * kThreads;
+        if(ou >= nblk * P) break;
+        const uint32_t sb = ou / P;
+        for(uint32_t r = nblk + f[u] - sb; r + sb + 1 < nblk + l[u]; ++r) {   // the other lists of the block
+          const Piece add = *reinterpret_cast<const Piece*>(s_row + r * LDW + (ou % P) * W);
+#pragma unroll
+          for(int q = 0; q < W; ++q) sum[u].v[q] += add.v[q];
+        }
+        dst[ou] = sum[u];
+      }
+    }
+  }
+  if constexpr(RHS) {
+    // four lanes per rhs entry, each a quarter of the row's lists (strided), added by shuffles
+    const uint32_t h = t & 3u;
+    for(uint32_t o = t >> 2; o < (nrows * NEQ + 15) / 16 * 16; o += kThreads / 4) {   // whole waves
+      const uint32_t oo = min(o, nrows * NEQ - 1), row = oo / NEQ, r = oo % NEQ;
+      const uint32_t qe = s_rowfirst[row + 1];
+      R sum = R(0);
+      for(uint32_t q = s_rowfirst[row] + h; q < qe; q += 4) sum -= s_rhs[q * NEQ + r];
+      sum += __shfl_xor(sum, 1, 64);
+      sum += __shfl_xor(sum, 2, 64);
+      if(h == 0 && o < nrows * NEQ) g.rhs[(uint64_t)r0 * NEQ + o] = (double)sum;
+    }
+  }
+}
+
+template<int D, typename R, bool RHS>
+__global__ __launch_bounds__(kThreads, sizeof(R) == sizeof(float) ? 4 : 3) void k_assemble_lists(AsmArgs g)
+{
+  extern __shared__ double4 s_dyn[];
+  assemble_lists_wg<D, R, RHS>(g, xcd_order(blockIdx.x, gridDim.x), reinterpret_cast<unsigned char*>(s_dyn));
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -784,11 +1041,12 @@ __global__ void k_batch_pack(const BatchHeader* __restrict__ hd, const BatchEntr
 __global__ __launch_bounds__(kThreads) void k_batch_assemble(const BatchHeader* __restrict__ hd,
                                                               const BatchEntry* __restrict__ e)
 {
+  extern __shared__ double4 s_dyn[];
   const uint32_t total = hd->total_wg, n = hd->n_cases;
   for(uint32_t task = blockIdx.x; task < total; task += gridDim.x) {
     __syncthreads();   // the previous task's LDS reads are done
     const uint32_t c = batch_find(e, n, task, true);
-    assemble_wg<SpecP1<3, float>, float, float, false>(e[c].g, task - e[c].wg_begin);
+    assemble_lists_wg<3, float, false>(e[c].g, task - e[c].wg_begin, reinterpret_cast<unsigned char*>(s_dyn));
   }
 }
 
@@ -904,32 +1162,26 @@ void launch(const AsmArgs& g, const Lss& L)
 {
   Context& c = *L.ctx;
   timer_begin(c, CF3HIP_KERNEL_ASSEMBLY);
-  hipLaunchKernelGGL((k_assemble<Op, R, VR, RHS, false>), dim3(L.n_wg), dim3(kThreads), 0, c.stream, g);
+  hipLaunchKernelGGL((k_assemble<Op, R, VR, RHS>), dim3(L.n_wg), dim3(kThreads), 0, c.stream, g);
   HIP_OK(hipGetLastError());
   timer_end(c, CF3HIP_KERNEL_ASSEMBLY);
 }
 
-// specialised simplex kernels: the FP64 kernel is node-staged when the system has the staging
-// structures (measured at 64^3 tetrahedra: 0.437-0.448 ms against 0.451-0.463 ms unstaged, 144
-// instead of 164 VGPRs).  The FP32 kernel stays unstaged: it already runs 5 waves per SIMD, and the
-// staging copy and its barrier cost more than the gathers it saves (0.260 ms against 0.237-0.249 ms).
-template<class Op, typename R, typename VR, bool RHS>
+// specialised simplices: by block lists; a system without plans (a workgroup that touches more than
+// kPlanNodes nodes, or a node with too many elements) takes the staged reduction
+template<int D, typename R, bool RHS>
 void launch_spec(const AsmArgs& g, const Lss& L)
 {
-  if constexpr(sizeof(R) != sizeof(double)) {
-    launch<Op, R, VR, RHS>(g, L);
-  } else {
-    if(!L.staged) {
-      launch<Op, R, VR, RHS>(g, L);
-      return;
-    }
-    Context& c = *L.ctx;
-    const size_t lds = sizeof(double4) * 3 * (size_t)L.wg_nodes_max;
-    timer_begin(c, CF3HIP_KERNEL_ASSEMBLY);
-    hipLaunchKernelGGL((k_assemble<Op, R, VR, RHS, true>), dim3(L.n_wg), dim3(kThreads), lds, c.stream, g);
-    HIP_OK(hipGetLastError());
-    timer_end(c, CF3HIP_KERNEL_ASSEMBLY);
+  if(!g.plan) {
+    launch<SpecP1<D, R>, R, R, RHS>(g, L);
+    return;
   }
+  Context& c = *L.ctx;
+  const size_t lds = PlanLayout<D, R>::lds_bytes(RHS, L.plan_nodes, L.plan_elems, L.plan_lists);
+  timer_begin(c, CF3HIP_KERNEL_ASSEMBLY);
+  hipLaunchKernelGGL((k_assemble_lists<D, R, RHS>), dim3(L.n_plan), dim3(kThreads), lds, c.stream, g);
+  HIP_OK(hipGetLastError());
+  timer_end(c, CF3HIP_KERNEL_ASSEMBLY);
 }
 
 __global__ void k_clear_flag(int* f) { f[0] = 0; }
@@ -960,10 +1212,9 @@ AsmArgs make_args(Lss& L, Fields& F, const cf3hip_ns_params& prm, bool pack = tr
   g.inc_pos = L.inc_pos.as<uint8_t>();
   g.blk_beg = L.blk_beg.as<uint8_t>();
   g.blk_acc = L.blk_acc.as<uint16_t>();
-  if(L.staged) {
-    g.wg_head = L.wg_head.as<uint32_t>();
-    g.wg_nodes = L.wg_nodes.as<uint32_t>();
-    g.inc_loc = L.inc_loc.as<uint32_t>();
+  if(L.n_plan) {
+    g.plan = L.plan.as<unsigned char>();
+    g.plan_nodes = L.plan_nodes; g.plan_elems = L.plan_elems; g.plan_lists = L.plan_lists;
   }
   g.rho = prm.rho; g.inv_rho = 1. / prm.rho;
   g.dt = prm.dt; g.theta = prm.theta; g.thq = prm.theta * (1. / prm.theta);
@@ -1030,11 +1281,11 @@ void assemble(Lss& L, Fields& F, const cf3hip_ns_params& prm)
   if(is_cell(M.etype)) {
     launch_hex(g, L, fp32 ? 1 : 0);
   } else if(spec && M.etype == CF3HIP_TETRA3D) {
-    if(fp32) launch_spec<SpecP1<3, float>, float, float, false>(g, L);
-    else launch_spec<SpecP1<3, double>, double, double, true>(g, L);
+    if(fp32) launch_spec<3, float, false>(g, L);
+    else launch_spec<3, double, true>(g, L);
   } else if(spec && M.etype == CF3HIP_TRIAG2D) {
-    if(fp32) launch_spec<SpecP1<2, float>, float, float, false>(g, L);
-    else launch_spec<SpecP1<2, double>, double, double, true>(g, L);
+    if(fp32) launch_spec<2, float, false>(g, L);
+    else launch_spec<2, double, true>(g, L);
   } else if(M.etype == CF3HIP_TETRA3D) {
     if(fp32) launch<GenericP1<3>, double, float, false>(g, L);
     else launch<GenericP1<3>, double, double, true>(g, L);
@@ -1087,6 +1338,7 @@ void batch_assemble(Batch& B, uint32_t n, Lss* const* L, Fields* const* F, const
   BatchHeader* hd = reinterpret_cast<BatchHeader*>(B.host_table);
   BatchEntry* ent = reinterpret_cast<BatchEntry*>(static_cast<char*>(B.host_table) + kBatchHeaderBytes);
   uint32_t wg = 0, nodes = 0;
+  size_t lds = 16384;   // LDS of the captured launch; systems that need more capture it again
   for(uint32_t i = 0; i < n; ++i) {
     Lss& Li = *L[i];
     Fields& Fi = *F[i];
@@ -1094,7 +1346,7 @@ void batch_assemble(Batch& B, uint32_t n, Lss* const* L, Fields* const* F, const
       CF3_THROW(CF3HIP_ERR_NOT_IMPLEMENTED, "batched assembly takes tetrahedral systems with the specialised kernel");
     if(!Li.has_fp32) CF3_THROW(CF3HIP_ERR_NOT_CREATED, "batched FP32 assembly needs cf3hip_lss_enable_fp32");
     if(Li.periodic) CF3_THROW(CF3HIP_ERR_NOT_IMPLEMENTED, "batched assembly takes systems without periodic links");
-    if((uint64_t)wg + Li.n_wg > 0xffffffffull || (uint64_t)nodes + Li.n_nodes > 0xffffffffull)
+    if((uint64_t)wg + Li.n_plan > 0xffffffffull || (uint64_t)nodes + Li.n_nodes > 0xffffffffull)
       CF3_THROW(CF3HIP_ERR_LIMIT, "batch too large");
     // ZeroLSS: forget the conditions of the previous step (mask cleared on the batch stream)
     Li.bc_host.clear();
@@ -1119,27 +1371,41 @@ void batch_assemble(Batch& B, uint32_t n, Lss* const* L, Fields* const* F, const
     ent[i].wg_begin = wg;
     ent[i].node_begin = nodes;
     ent[i].n_nodes = Li.n_nodes;
-    wg += Li.n_wg;
+    wg += Li.n_plan;
     nodes += Li.n_nodes;
+    if(Li.n_plan)
+      lds = std::max(lds, PlanLayout<3, float>::lds_bytes(false, Li.plan_nodes, Li.plan_elems, Li.plan_lists));
   }
   hd->n_cases = n;
   hd->total_wg = n ? wg : 0;
   hd->total_nodes = n ? nodes : 0;
   HIP_OK(hipMemcpyAsync(B.table.ptr, B.host_table, kBatchHeaderBytes + sizeof(BatchEntry) * (n ? n : 1),
                         hipMemcpyHostToDevice, B.stream));
+  if(B.exec && lds > B.lds) {
+    HIP_OK(hipGraphExecDestroy(B.exec));
+    HIP_OK(hipGraphDestroy(B.graph));
+    B.exec = nullptr;
+    B.graph = nullptr;
+  }
   if(!B.exec) {
+    B.lds = lds;
     // the two launches read the table from device memory, so one capture serves every later batch
     const BatchHeader* dh = B.table.as<BatchHeader>();
     const BatchEntry* de = reinterpret_cast<const BatchEntry*>(B.table.as<char>() + kBatchHeaderBytes);
     hipGraph_t graph = nullptr;
     HIP_OK(hipStreamBeginCapture(B.stream, hipStreamCaptureModeThreadLocal));
     hipLaunchKernelGGL(k_batch_pack, dim3(kBatchPackGrid), dim3(256), 0, B.stream, dh, de);
-    hipLaunchKernelGGL(k_batch_assemble, dim3(kBatchAsmGrid), dim3(kThreads), 0, B.stream, dh, de);
+    hipLaunchKernelGGL(k_batch_assemble, dim3(kBatchAsmGrid), dim3(kThreads), lds, B.stream, dh, de);
     HIP_OK(hipStreamEndCapture(B.stream, &graph));
     HIP_OK(hipGraphInstantiate(&B.exec, graph, nullptr, nullptr, 0));
     B.graph = graph;
   }
   HIP_OK(hipGraphLaunch(B.exec, B.stream));
+  for(uint32_t i = 0; i < n; ++i)   // systems without plans: the staged reduction, after the pack
+    if(!L[i]->n_plan)
+      hipLaunchKernelGGL((k_assemble<SpecP1<3, float>, float, float, false>), dim3(L[i]->n_wg), dim3(kThreads), 0,
+                         B.stream, ent[i].g);
+  HIP_OK(hipGetLastError());
   HIP_OK(hipStreamSynchronize(B.stream));
   for(uint32_t i = 0; i < n; ++i) check_status(*L[i]->ctx);
 }

@@ -23,9 +23,8 @@ struct AsmArgs {
   const uint8_t* inc_pos;   // per incidence: staging row of its block in pass b (byte b)
   const uint8_t* blk_beg;   // per block: first staging row of pass p (byte p)
   const uint16_t* blk_acc;  // per block: first accumulator thread (low byte), accumulator count (high byte)
-  const uint32_t* wg_head;  // node staging: per workgroup r0, r1, i0, i1, b0, b1, n0, n1
-  const uint32_t* wg_nodes; // node staging: distinct nodes of each workgroup
-  const uint32_t* inc_loc;  // node staging: per incidence the local indices of its element's nodes
+  const unsigned char* plan; // specialised simplices: assembly plans (null: staged reduction only)
+  uint32_t plan_nodes, plan_elems, plan_lists;
   void* values;
   double* rhs;
   const double* xt;    // matrix-free residual: x with constrained columns set to their first value
@@ -81,6 +80,25 @@ __device__ __forceinline__ double tet_volume_ref(const double X[4][3])
           x3*y1*z2 + x0*y3*z2 - x1*y3*z2 - x1*y0*z3 + x2*y0*z3 +
           x0*y1*z3 - x2*y1*z3 - x0*y2*z3 + x1*y2*z3) / 6.;
 }
+
+// 1 / x and 1 / sqrt(x) for positive normal x by Newton steps from the hardware estimates: within an ulp or
+// two, in 5 and 9 FP64 instructions against 11 and about 25 of the correctly rounded division and root (the
+// element quantities take four of them per element).  Zero, negative, infinite and NaN arguments give what
+// the callers' Jacobian test reports or a NaN.
+__device__ __forceinline__ double reciprocal(double x)
+{
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(fma(-x, r, 1.), r, r);
+  return fma(fma(-x, r, 1.), r, r);
+}
+__device__ __forceinline__ float reciprocal(float x) { return 1.f / x; }
+__device__ __forceinline__ double inv_sqrt(double x)
+{
+  double r = __builtin_amdgcn_rsq(x);
+  r = fma(0.5 * r, fma(-x * r, r, 1.), r);
+  return fma(0.5 * r, fma(-x * r, r, 1.), r);
+}
+__device__ __forceinline__ float inv_sqrt(float x) { return 1.f / sqrtf(x); }
 
 // one LDS row of a staged element block: 16-byte aligned, odd number of 16-byte chunks (bank spread)
 template<typename VR, int NN>

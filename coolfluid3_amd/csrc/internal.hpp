@@ -91,7 +91,12 @@ constexpr int kMaxRedBlocks = 1024;
 // assembly workgroup: at most kAsmThreads incidences (one per thread) and kAsmThreads CSR blocks
 // (one owner thread per block); the row schedule of the system respects both
 constexpr int kAsmThreads = 128;
-constexpr uint32_t kMaxWgNodes = 255;   // distinct nodes per staged workgroup (one-byte local indices)
+// Assembly plans of the specialised simplex kernels (see sparsity.hip).  A workgroup holds at most
+// kPlanElems elements (its record kPlanElems stands for none), kAsmThreads block lists and kPlanNodes nodes.
+constexpr uint32_t kPlanElems = 127, kPlanNodes = 255;
+constexpr uint32_t plan_list_length(int k) { return k == 4 ? 6 : 3; }   // contributions per block list, at most
+constexpr uint32_t kPlanHeadBytes = 32;                                  // r0, rows, elements, nodes, blk0, blocks, lists, 0
+constexpr uint32_t plan_bytes(uint32_t ns) { return kPlanHeadBytes + 4 * ns + kAsmThreads * (4 + 8 + 2); }
 
 // ---------------------------------------------------------------------------------------------
 // mesh / system / fields
@@ -152,13 +157,12 @@ struct Lss {
   DevBuf inc_pos;       // uint8 n_elems*k*pos_stride
   DevBuf blk_beg;       // uint8 n_blocks*4
   DevBuf blk_acc;       // uint16 n_blocks: first accumulator thread (low byte) and count (high byte)
-  // node staging of the simplex kernels: each workgroup copies the records of the distinct nodes its
-  // elements touch into LDS once, and its incidences address them by local index
-  bool staged = false;  // built (simplices whose workgroups touch at most kMaxWgNodes nodes)
-  uint32_t wg_nodes_max = 0;
-  DevBuf wg_head;       // uint32 8 per workgroup: rows [r0, r1), incidences [i0, i1), blocks [b0, b1), nodes [n0, n1)
-  DevBuf wg_nodes;      // uint32: the distinct nodes of each workgroup, ascending
-  DevBuf inc_loc;       // uint32 n_elems*k: local indices (one byte per element node) of the element's nodes
+  // assembly plans of the specialised simplex kernels, one of plan_bytes(plan_nodes) per workgroup (empty:
+  // some row or workgroup does not fit, the staged reduction serves the system)
+  DevBuf plan;
+  uint32_t n_plan = 0;           // workgroups
+  uint32_t plan_nodes = 0;       // node slots of a plan (multiple of 4)
+  uint32_t plan_elems = 0, plan_lists = 0;   // most elements and block lists of a workgroup
   // Dirichlet conditions applied since the last reset (needed by the matrix-free FP64 residual):
   // per dof the first value (column elimination) and the last value (row / solution)
   std::unordered_map<uint64_t, std::pair<double, double> > bc_host;
@@ -247,6 +251,7 @@ struct Batch {
   void* host_table = nullptr;   // pinned mirror
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
+  size_t lds = 0;               // dynamic LDS of the captured assembly launch
 };
 
 // ---------------------------------------------------------------------------------------------

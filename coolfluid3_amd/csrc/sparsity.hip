@@ -150,6 +150,45 @@ __global__ void k_contrib_from_keys(const uint64_t* __restrict__ keys, uint64_t 
   contrib[j] = (uint16_t)((q << 4) | b);
 }
 
+// The block lists of one block, in order: groups of contributions with the same column mesh node (one group
+// unless the system is periodic), each split evenly over ceil(n / len) lists.  contrib: (q << 4 | b) in
+// (b, q) order, q relative to the block's row, whose incidences start at inc_row.  emit(at, count) is called
+// per list; at(m) is the position of its contribution m.
+template<class F>
+__device__ inline void for_block_lists(const uint16_t* contrib, uint32_t n, bool periodic, int k, uint32_t len,
+                                       const uint32_t* inc_row, const uint32_t* conn, F emit)
+{
+  if(!periodic) {
+    const uint32_t nl = (n + len - 1) / len;
+    for(uint32_t l = 0; l < nl; ++l) {
+      const uint32_t i0 = (n * l) / nl, i1 = (n * (l + 1)) / nl;   // at most len
+      emit([&](uint32_t m) { return i0 + m; }, i1 - i0);
+    }
+    return;
+  }
+  auto node = [&](uint32_t j) {
+    const uint32_t ea = inc_row[contrib[j] >> 4];
+    return conn[ea - ea % (uint32_t)k + (contrib[j] & 15u)];
+  };
+  uint32_t idx[8];
+  for(uint32_t j = 0; j < n; ++j) {
+    const uint32_t nd = node(j);
+    bool seen = false;
+    for(uint32_t i = 0; i < j && !seen; ++i) seen = node(i) == nd;
+    if(seen) continue;
+    uint32_t size = 0;
+    for(uint32_t i = j; i < n; ++i) size += node(i) == nd ? 1u : 0u;
+    const uint32_t nl = (size + len - 1) / len;
+    uint32_t i = j;
+    for(uint32_t l = 0; l < nl; ++l) {
+      const uint32_t take = (size * (l + 1)) / nl - (size * l) / nl;
+      for(uint32_t m = 0; m < take; ++i)
+        if(node(i) == nd) idx[m++] = i;
+      emit([&](uint32_t m) { return idx[m]; }, take);
+    }
+  }
+}
+
 // Accumulator threads of a block: enough that none sums more than kAccRows staged rows per pass.
 __global__ void k_block_acc(uint64_t n_blocks, int passes, const uint32_t* __restrict__ contrib_ptr,
                             const uint16_t* __restrict__ contrib, uint8_t* __restrict__ acc_cnt)
@@ -162,14 +201,25 @@ __global__ void k_block_acc(uint64_t n_blocks, int passes, const uint32_t* __res
   acc_cnt[s] = (uint8_t)max(1u, (mx + kAccRows - 1) / kAccRows);
 }
 
+// Per row: accumulator threads of the staged reduction (low half) and block lists (high half; simplices,
+// len > 0), each saturated at 0xffff (above any workgroup's limit).
 __global__ void k_row_acc(uint32_t n, const uint32_t* __restrict__ row_ptr, const uint8_t* __restrict__ acc_cnt,
+                          uint32_t len, bool periodic, int k, const uint32_t* __restrict__ contrib_ptr,
+                          const uint16_t* __restrict__ contrib, const uint32_t* __restrict__ inc_ptr,
+                          const uint32_t* __restrict__ inc, const uint32_t* __restrict__ conn,
                           uint32_t* __restrict__ row_acc)
 {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if(i >= n) return;
-  uint32_t a = 0;
-  for(uint32_t s = row_ptr[i]; s < row_ptr[i + 1]; ++s) a += acc_cnt[s];
-  row_acc[i] = a;
+  uint32_t a = 0, l = 0;
+  for(uint32_t s = row_ptr[i]; s < row_ptr[i + 1]; ++s) {
+    a += acc_cnt[s];
+    if(len == 0) continue;
+    const uint32_t c0 = contrib_ptr[s], nc = contrib_ptr[s + 1] - c0;
+    if(!periodic) l += (nc + len - 1) / len;
+    else for_block_lists(contrib + c0, nc, true, k, len, inc + inc_ptr[i], conn, [&](auto, uint32_t) { ++l; });
+  }
+  row_acc[i] = min(a, 0xffffu) | (min(l, 0xffffu) << 16);
 }
 
 // One workgroup per assembly workgroup: derive the staging maps from the contribution lists of its
@@ -226,34 +276,83 @@ __global__ __launch_bounds__(kAsmThreads) void k_stage_maps(int passes, int pos_
   }
 }
 
-// Node staging (simplices): the distinct nodes of the elements of one assembly workgroup, and per
-// incidence the local indices of its element's nodes in that list.  One workgroup per assembly
-// workgroup: the (at most kAsmThreads * 4) node ids are bitonic-sorted in LDS and de-duplicated.
-// FILL = false writes the count of each workgroup; FILL = true writes the list at nodes_ptr[wg] and
-// the local indices (byte m of inc_loc = local index of element node m).
-template<bool FILL>
-__global__ __launch_bounds__(kAsmThreads) void k_wg_nodes(int k, const uint32_t* __restrict__ wg_rows,
-                                                         const uint32_t* __restrict__ inc_ptr,
-                                                         const uint32_t* __restrict__ inc,
-                                                         const uint32_t* __restrict__ conn,
-                                                         const uint32_t* __restrict__ nodes_ptr,
-                                                         uint32_t* __restrict__ out, uint32_t* __restrict__ inc_loc)
+// ---- assembly plans of the specialised simplex kernels ----
+// A plan is what one workgroup of assemble_lists_wg reads, at a fixed stride, so that all its loads but
+// those of the node records start at once:
+//   head   r0, rows, elements, nodes, blk0, blocks, block lists, 0
+//   nodes  uint32[ns]: the distinct mesh nodes of its elements, ascending, the last one repeated
+//   loc    uint32[128]: per element the local indices of its nodes, byte m = node m
+//   lo     uint64[128], hi uint16[128]: the block lists, in block order.  Entry i (11 bits) = element << 4 |
+//          a << 2 | b, the row and column local nodes; entries 0-4 at bits 11 i of lo, entry 5 in hi;
+//          unused entries name element `elements`.  lo bits 55-62: local index of the column node, bit 63:
+//          first list of a block; hi bit 15: first list of a row.
+// All contributions of a list have the same column mesh node (under periodic links a block may have several).
+// A workgroup takes consecutive rows while its distinct elements, lists and rows fit; element sharing between
+// neighbouring rows is what makes a workgroup of elements cheaper than one of (element, row) incidences.
+
+// Rows one wave partitions in order; a workgroup never spans two segments.  Long segments leave few short
+// workgroups at their ends, short ones keep the partition of a small mesh from being one long chain.
+inline uint32_t plan_segment(uint64_t rows) { return rows < 65536 ? 63 : 252; }
+
+// Distance in rows from each incidence's row back to the nearest earlier row of its element (255: none
+// within 254): the element is new to a workgroup that starts at r0 exactly when that row is before r0.
+__global__ void k_inc_back(uint64_t nek, int k, const uint32_t* __restrict__ inc, const uint32_t* __restrict__ rconn,
+                           uint8_t* __restrict__ back)
 {
-  constexpr uint32_t S = kAsmThreads * 4;
-  __shared__ uint32_t s[S];
-  __shared__ uint32_t s_u[S];
-  __shared__ uint32_t s_cnt[kAsmThreads + 1];
-  const uint32_t r0 = wg_rows[blockIdx.x], r1 = wg_rows[blockIdx.x + 1];
-  const uint32_t i0 = inc_ptr[r0], ninc = inc_ptr[r1] - i0;
-  const uint32_t t = threadIdx.x;
-  uint32_t mine[4] = {0xffffffffu, 0xffffffffu, 0xffffffffu, 0xffffffffu};
-  if(t < ninc) {
-    const uint64_t e = inc[i0 + t] / (uint32_t)k;
-    for(int m = 0; m < k; ++m) mine[m] = conn[e * k + m];
+  const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if(t >= nek) return;
+  const uint32_t ea = inc[t], a = ea % (uint32_t)k;
+  const uint32_t* en = rconn + (ea - a);
+  const uint32_t row = en[a];
+  uint32_t d = 255;
+  for(uint32_t m = 0; m < (uint32_t)k; ++m) {
+    // a periodic element may hold a row twice: its second node there is never new
+    if(en[m] < row) d = min(d, row - en[m]);
+    else if(en[m] == row && m < a) d = 0;
   }
-  for(int m = 0; m < 4; ++m) s[m * kAsmThreads + t] = mine[m];
-  __syncthreads();
-  // bitonic sort, ascending (unused slots hold 0xffffffff and sort last)
+  back[t] = (uint8_t)d;
+}
+
+// One wave per segment of rows: start[r] = 1 where a workgroup starts.  fits stays 0 unless a row alone
+// exceeds a limit.
+__global__ __launch_bounds__(64) void k_plan_partition(uint32_t N, uint32_t segment, const uint32_t* __restrict__ inc_ptr,
+                                                       const uint8_t* __restrict__ back,
+                                                       const uint32_t* __restrict__ row_lists,
+                                                       uint8_t* __restrict__ start, int* __restrict__ misfit)
+{
+  const uint32_t b = blockIdx.x * segment, e = min(N, b + segment);
+  const uint32_t lane = threadIdx.x;
+  uint32_t r0 = b, ne = 0, nl = 0;
+  for(uint32_t r = b; r < e; ++r) {
+    const uint32_t i0 = inc_ptr[r], i1 = inc_ptr[r + 1], lists = row_lists[r] >> 16;
+    uint32_t fresh = 0, own = 0;   // elements new to the open workgroup, and to one that starts here
+    for(uint32_t i = i0 + lane; i - lane < i1; i += 64) {
+      const uint32_t d = i < i1 ? back[i] : 0;
+      fresh += (uint32_t)__popcll(__ballot(i < i1 && d > r - r0));
+      own += (uint32_t)__popcll(__ballot(i < i1 && d > 0));
+    }
+    if(own > kPlanElems || lists > (uint32_t)kAsmThreads) {
+      if(lane == 0) misfit[0] = 1;
+      return;
+    }
+    const bool open = r == b || ne + fresh > kPlanElems || nl + lists > (uint32_t)kAsmThreads ||
+                      r - r0 >= (uint32_t)kAsmThreads;
+    if(open) { r0 = r; ne = own; nl = lists; }
+    else { ne += fresh; nl += lists; }
+    if(lane == 0) start[r] = open ? 1 : 0;
+  }
+}
+
+__global__ void k_iota(uint32_t n, uint32_t* __restrict__ out)
+{
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if(i < n) out[i] = i;
+}
+
+// ascending bitonic sort of S (a power of two) LDS values
+template<uint32_t S>
+__device__ inline void lds_sort(uint32_t* s, uint32_t t)
+{
   for(uint32_t size = 2; size <= S; size <<= 1)
     for(uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
       for(uint32_t p = t; p < S / 2; p += kAsmThreads) {
@@ -263,50 +362,192 @@ __global__ __launch_bounds__(kAsmThreads) void k_wg_nodes(int k, const uint32_t*
       }
       __syncthreads();
     }
-  // distinct values: thread t takes positions 4t .. 4t+3
-  uint32_t f = 0;
-  for(uint32_t m = 0; m < 4; ++m) {
-    const uint32_t i = 4 * t + m;
-    if(s[i] != 0xffffffffu && (i == 0 || s[i] != s[i - 1])) f |= 1u << m;
+}
+
+// position of v in the ascending s[0, n), which holds it
+__device__ inline uint32_t lds_find(const uint32_t* s, uint32_t n, uint32_t v)
+{
+  uint32_t lo = 0, hi = n;
+  while(hi - lo > 1) {
+    const uint32_t mid = (lo + hi) >> 1;
+    if(s[mid] <= v) lo = mid; else hi = mid;
   }
-  s_cnt[t] = __popc(f);
+  return lo;
+}
+
+// exclusive scan of one value per thread; total in every thread
+__device__ inline uint32_t wg_scan(uint32_t v, uint32_t* s_wave, uint32_t t, uint32_t& total)
+{
+  constexpr uint32_t W = kAsmThreads / 64;
+  uint32_t x = v;
+#pragma unroll
+  for(uint32_t off = 1; off < 64; off <<= 1) {
+    const uint32_t y = __shfl_up(x, off, 64);
+    if((t & 63u) >= off) x += y;
+  }
+  if((t & 63u) == 63u) s_wave[t >> 6] = x;
   __syncthreads();
+  uint32_t before = 0;
+  total = 0;
+  for(uint32_t w = 0; w < W; ++w) {
+    if(w < (t >> 6)) before += s_wave[w];
+    total += s_wave[w];
+  }
+  __syncthreads();
+  return before + x - v;
+}
+
+// slot of key in an open-addressing table of T (a power of two) LDS words, 0xffffffff = free; fresh is set
+// for the one thread that put it there
+template<uint32_t T>
+__device__ inline uint32_t lds_insert(uint32_t* table, uint32_t key, bool& fresh)
+{
+  uint32_t h = (key * 2654435761u) >> 16;
+  for(;; ++h) {
+    h &= T - 1;
+    const uint32_t old = atomicCAS(&table[h], 0xffffffffu, key);
+    if(old == 0xffffffffu || old == key) { fresh = old != key; return h; }
+  }
+}
+
+// The plan of one workgroup.  most[0..2]: largest node, element and list count seen; a plan with more than
+// ns nodes is left unfinished (the caller runs again with more slots).
+__global__ __launch_bounds__(kAsmThreads) void k_plan_fill(uint32_t N, uint32_t n_plan, int k, uint32_t len, bool periodic,
+                                                           uint32_t ns, const uint32_t* __restrict__ wg_start,
+                                                           const uint32_t* __restrict__ row_ptr,
+                                                           const uint32_t* __restrict__ inc_ptr,
+                                                           const uint32_t* __restrict__ inc,
+                                                           const uint8_t* __restrict__ back,
+                                                           const uint32_t* __restrict__ rconn,
+                                                           const uint32_t* __restrict__ conn,
+                                                           const uint32_t* __restrict__ contrib_ptr,
+                                                           const uint16_t* __restrict__ contrib,
+                                                           unsigned char* __restrict__ plans, uint32_t* __restrict__ most)
+{
+  constexpr uint32_t S = kAsmThreads * 4;   // at least the nodes and the incidences of kPlanElems elements
+  __shared__ uint32_t s_etab[2 * kAsmThreads], s_ntab[2 * S], s_uniq[S], s_wave[kAsmThreads / 64];
+  __shared__ uint32_t s_elem[kAsmThreads], s_loc[kAsmThreads];
+  __shared__ uint8_t s_eidx[2 * kAsmThreads];
+  __shared__ uint16_t s_inc[S];             // per incidence: element << 2 | a
+  __shared__ uint16_t s_contrib[4 * S];     // the contributions of the workgroup's blocks
+  const uint32_t wg = blockIdx.x, t = threadIdx.x;
+  const uint32_t r0 = wg_start[wg], r1 = wg + 1 < n_plan ? wg_start[wg + 1] : N;
+  const uint32_t i0 = inc_ptr[r0], ninc = inc_ptr[r1] - i0;
+  const uint32_t blk0 = row_ptr[r0], nblk = row_ptr[r1] - blk0;
+  for(uint32_t j = t; j < 2 * kAsmThreads; j += kAsmThreads) s_etab[j] = 0xffffffffu;
+  for(uint32_t j = t; j < 2 * S; j += kAsmThreads) s_ntab[j] = 0xffffffffu;
+  __syncthreads();
+  // distinct elements, in the order of their first incidence
+  uint32_t ne = 0;
+  for(uint32_t base = 0; base < ninc; base += kAsmThreads) {
+    const uint32_t i = i0 + base + t;
+    bool fresh = false, put;
+    uint32_t ea = 0;
+    if(base + t < ninc) {
+      ea = inc[i];
+      fresh = back[i] > rconn[ea] - r0;
+    }
+    uint32_t total;
+    const uint32_t at = ne + wg_scan(fresh ? 1u : 0u, s_wave, t, total);
+    if(fresh) {
+      s_elem[at] = ea / (uint32_t)k;
+      s_eidx[lds_insert<2 * kAsmThreads>(s_etab, ea / (uint32_t)k, put)] = (uint8_t)at;
+    }
+    ne += total;
+  }
+  __syncthreads();
+  // distinct nodes, ascending
+  uint32_t mine[4] = {0, 0, 0, 0}, f = 0, nn;
+  if(t < ne)
+    for(int m = 0; m < k; ++m) {
+      bool put;
+      mine[m] = conn[(uint64_t)s_elem[t] * k + m];
+      (void)lds_insert<2 * S>(s_ntab, mine[m], put);
+      f |= put ? 1u << m : 0u;
+    }
+  uint32_t o = wg_scan((uint32_t)__popc(f), s_wave, t, nn);
+  for(uint32_t j = t; j < S; j += kAsmThreads) s_uniq[j] = 0xffffffffu;
+  __syncthreads();
+  for(int m = 0; m < 4; ++m)
+    if(f & (1u << m)) s_uniq[o++] = mine[m];
+  __syncthreads();
+  if(nn <= kAsmThreads) lds_sort<kAsmThreads>(s_uniq, t);
+  else lds_sort<S>(s_uniq, t);
+  uint32_t packed = 0;
+  if(t < ne)
+    for(int m = 0; m < k; ++m) packed |= lds_find(s_uniq, nn, mine[m]) << (8 * m);
+  s_loc[t] = packed;
+  for(uint32_t i = t; i < ninc; i += kAsmThreads) {
+    const uint32_t ea = inc[i0 + i];
+    bool put;
+    s_inc[i] = (uint16_t)((uint32_t)s_eidx[lds_insert<2 * kAsmThreads>(s_etab, ea / (uint32_t)k, put)] << 2 |
+                          ea % (uint32_t)k);
+  }
+  const uint32_t cb = contrib_ptr[blk0], nct = contrib_ptr[blk0 + nblk] - cb;
+  for(uint32_t i = t; i < nct; i += kAsmThreads) s_contrib[i] = contrib[cb + i];
+  __syncthreads();
+  // block lists
+  uint32_t nc = 0, ib = 0, cnt = 0, row = r0;
+  const uint16_t* ctr = s_contrib;
+  if(t < nblk) {
+    uint32_t hi = r1;
+    while(hi - row > 1) {
+      const uint32_t mid = (row + hi) >> 1;
+      if(row_ptr[mid] <= blk0 + t) row = mid; else hi = mid;
+    }
+    ib = inc_ptr[row];
+    const uint32_t c0 = contrib_ptr[blk0 + t];
+    ctr += c0 - cb;
+    nc = contrib_ptr[blk0 + t + 1] - c0;
+    for_block_lists(ctr, nc, periodic, k, len, inc + ib, conn, [&](auto, uint32_t) { ++cnt; });
+  }
+  uint32_t nlists;
+  const uint32_t first = wg_scan(cnt, s_wave, t, nlists);
+  if(t < 3) {
+    // every workgroup's atomics on the same words would take longer than all the rest of the kernel: only
+    // those that raise the maximum seen (a stale value costs an atomic, never a maximum)
+    const uint32_t v = t == 0 ? nn : t == 1 ? ne : nlists;
+    if(v > *static_cast<volatile const uint32_t*>(&most[t])) atomicMax(&most[t], v);
+  }
+  if(nn > ns) return;
+  unsigned char* plan = plans + (uint64_t)wg * plan_bytes(ns);
+  uint32_t* head = reinterpret_cast<uint32_t*>(plan);
+  uint32_t* nodes = reinterpret_cast<uint32_t*>(plan + kPlanHeadBytes);
+  uint32_t* loc = nodes + ns;
+  uint64_t* lo = reinterpret_cast<uint64_t*>(loc + kAsmThreads);
+  uint16_t* hi = reinterpret_cast<uint16_t*>(lo + kAsmThreads);
   if(t == 0) {
-    uint32_t run = 0;
-    for(uint32_t j = 0; j < kAsmThreads; ++j) {
-      const uint32_t c = s_cnt[j];
-      s_cnt[j] = run;
-      run += c;
-    }
-    s_cnt[kAsmThreads] = run;
+    head[0] = r0; head[1] = r1 - r0; head[2] = ne; head[3] = nn;
+    head[4] = blk0; head[5] = nblk; head[6] = nlists; head[7] = 0;
   }
-  __syncthreads();
-  const uint32_t total = s_cnt[kAsmThreads];
-  if constexpr(!FILL) {
-    if(t == 0) out[blockIdx.x] = total;
-  } else {
-    uint32_t o = s_cnt[t];
-    const uint32_t base = nodes_ptr[blockIdx.x];
-    for(uint32_t m = 0; m < 4; ++m)
-      if(f & (1u << m)) {
-        s_u[o] = s[4 * t + m];
-        out[base + o] = s[4 * t + m];
-        ++o;
-      }
-    __syncthreads();
-    if(t < ninc) {
-      uint32_t packed = 0;
-      for(int m = 0; m < k; ++m) {
-        uint32_t lo = 0, hi = total;   // s_u[lo] == mine[m]
-        while(hi - lo > 1) {
-          const uint32_t mid = (lo + hi) >> 1;
-          if(s_u[mid] <= mine[m]) lo = mid; else hi = mid;
+  for(uint32_t j = t; j < ns; j += kAsmThreads) nodes[j] = s_uniq[min(j, nn - 1)];
+  loc[t] = packed;
+  if(t < nblk) {
+    uint32_t at = first;
+    bool blk_first = true;
+    const bool row_first = blk0 + t == row_ptr[row];
+    const uint16_t* binc = s_inc + (ib - i0);
+    for_block_lists(ctr, nc, periodic, k, len, inc + ib, conn, [&](auto pos, uint32_t n) {
+      uint64_t w = blk_first ? 1ull << 63 : 0;
+      uint32_t h = blk_first && row_first ? 0x8000u : 0;
+#pragma unroll
+      for(uint32_t m = 0; m < 6; ++m) {
+        uint32_t entry = ne << 4;
+        if(m < n) {
+          const uint32_t c = ctr[pos(m)], b = c & 15u, ea = binc[c >> 4];
+          entry = ea << 2 | b;
+          if(m == 0) w |= (uint64_t)((s_loc[ea >> 2] >> (8 * b)) & 255u) << 55;
         }
-        packed |= lo << (8 * m);
+        if(m < 5) w |= (uint64_t)entry << (11 * m);
+        else h |= entry;
       }
-      inc_loc[i0 + t] = packed;
-    }
+      lo[at] = w;
+      hi[at] = (uint16_t)h;
+      ++at;
+      blk_first = false;
+    });
   }
+  for(uint32_t j = nlists + t; j < kAsmThreads; j += kAsmThreads) { lo[j] = 0; hi[j] = 0; }
 }
 
 // out[i] = map[in[i]]
@@ -446,12 +687,15 @@ void build_element_structures(Lss& L)
     HIP_OK(hipGetLastError());
   }
   // accumulator threads per block and per row
+  const uint32_t list_len = q1 ? 0 : plan_list_length((int)k);
   acc_cnt.alloc(&c, L.n_blocks);
   row_acc.alloc(&c, sizeof(uint32_t) * N);
   hipLaunchKernelGGL(k_block_acc, dim3(grid_for(L.n_blocks, 256)), dim3(256), 0, c.stream, L.n_blocks, L.passes,
                      contrib_ptr.as<uint32_t>(), contrib.as<uint16_t>(), acc_cnt.as<uint8_t>());
   hipLaunchKernelGGL(k_row_acc, dim3(grid_for(N, 256)), dim3(256), 0, c.stream, (uint32_t)N, L.row_ptr.as<uint32_t>(),
-                     acc_cnt.as<uint8_t>(), row_acc.as<uint32_t>());
+                     acc_cnt.as<uint8_t>(), list_len, L.periodic, (int)k, contrib_ptr.as<uint32_t>(),
+                     contrib.as<uint16_t>(), L.inc_ptr.as<uint32_t>(), L.inc.as<uint32_t>(), M.conn.as<uint32_t>(),
+                     row_acc.as<uint32_t>());
   HIP_OK(hipGetLastError());
 
   // ---- host-side schedule of rows into assembly workgroups (structure only) ----
@@ -470,7 +714,7 @@ void build_element_structures(Lss& L)
     uint64_t ninc = 0, nacc = 0;
     while(r1 < N) {
       const uint64_t di = inc_ptr[r1 + 1] - inc_ptr[r1];
-      const uint64_t da = racc[r1];
+      const uint64_t da = racc[r1] & 0xffffu;
       if(di > inc_limit || da > (uint64_t)kAsmThreads)
         CF3_THROW(CF3HIP_ERR_LIMIT, "node " + std::to_string(r1) + " has " + std::to_string(di) +
                                         " incident elements and needs " + std::to_string(da) +
@@ -500,45 +744,53 @@ void build_element_structures(Lss& L)
                      L.inc_pos.as<uint8_t>(), L.blk_beg.as<uint8_t>(), L.blk_acc.as<uint16_t>());
   HIP_OK(hipGetLastError());
 
-  // ---- node staging (simplices) ----
-  L.staged = false;
-  if(!q1 && L.n_wg > 0) {
-    DevBuf counts;
-    counts.alloc(&c, sizeof(uint32_t) * L.n_wg);
-    hipLaunchKernelGGL(k_wg_nodes<false>, dim3(L.n_wg), dim3(kAsmThreads), 0, c.stream, (int)k,
-                       L.wg_rows.as<uint32_t>(), L.inc_ptr.as<uint32_t>(), L.inc.as<uint32_t>(), M.conn.as<uint32_t>(),
-                       (const uint32_t*)nullptr, counts.as<uint32_t>(), (uint32_t*)nullptr);
-    HIP_OK(hipGetLastError());
-    std::vector<uint32_t> cnt(L.n_wg), row_ptr(N + 1);
-    HIP_OK(hipMemcpyAsync(cnt.data(), counts.ptr, sizeof(uint32_t) * L.n_wg, hipMemcpyDeviceToHost, c.stream));
-    HIP_OK(hipMemcpyAsync(row_ptr.data(), L.row_ptr.ptr, sizeof(uint32_t) * (N + 1), hipMemcpyDeviceToHost, c.stream));
+  // ---- assembly plans (simplices) ----
+  if(!q1 && N > 0) {
+    // one allocation: info (n_plan, misfit, most[3]), row numbers, workgroup starts, start flags, back
+    DevBuf scratch, temp;
+    scratch.alloc(&c, 32 + 9 * N + nek);
+    uint32_t* inf = scratch.as<uint32_t>();
+    uint32_t *rows = inf + 8, *starts = rows + N;
+    uint8_t* flag = reinterpret_cast<uint8_t*>(starts + N);
+    uint8_t* back = flag + N;
+    uint32_t host[5] = {0, 0, 0, 0, 0};
+    HIP_OK(hipMemcpyAsync(inf, host, sizeof(host), hipMemcpyHostToDevice, c.stream));
+    hipLaunchKernelGGL(k_inc_back, dim3(grid_for(nek, 256)), dim3(256), 0, c.stream, nek, (int)k, L.inc.as<uint32_t>(),
+                       conn, back);
+    hipLaunchKernelGGL(k_plan_partition, dim3(grid_for(N, plan_segment(N))), dim3(64), 0, c.stream, (uint32_t)N,
+                       plan_segment(N),
+                       L.inc_ptr.as<uint32_t>(), back, row_acc.as<uint32_t>(), flag,
+                       reinterpret_cast<int*>(inf + 1));
+    hipLaunchKernelGGL(k_iota, dim3(grid_for(N, 256)), dim3(256), 0, c.stream, (uint32_t)N, rows);
+    size_t temp_bytes = 0;
+    HIP_OK(hipcub::DeviceSelect::Flagged(nullptr, temp_bytes, rows, flag,
+                                         starts, inf, (int)N, c.stream));
+    temp.alloc(&c, std::max<size_t>(temp_bytes, 16));
+    HIP_OK(hipcub::DeviceSelect::Flagged(temp.ptr, temp_bytes, rows, flag,
+                                         starts, inf, (int)N, c.stream));
+    HIP_OK(hipMemcpyAsync(host, inf, sizeof(host), hipMemcpyDeviceToHost, c.stream));
     HIP_OK(hipStreamSynchronize(c.stream));
-    const uint32_t mx = *std::max_element(cnt.begin(), cnt.end());
-    if(mx <= kMaxWgNodes) {
-      std::vector<uint32_t> nptr(L.n_wg + 1), head((size_t)L.n_wg * 8);
-      nptr[0] = 0;
-      for(uint32_t w = 0; w < L.n_wg; ++w) nptr[w + 1] = nptr[w] + cnt[w];
-      for(uint32_t w = 0; w < L.n_wg; ++w) {
-        const uint32_t r0 = wg[w], r1 = wg[w + 1];
-        uint32_t* h = &head[(size_t)w * 8];
-        h[0] = r0; h[1] = r1; h[2] = inc_ptr[r0]; h[3] = inc_ptr[r1];
-        h[4] = row_ptr[r0]; h[5] = row_ptr[r1]; h[6] = nptr[w]; h[7] = nptr[w + 1];
-      }
-      DevBuf dptr;
-      dptr.alloc(&c, sizeof(uint32_t) * (L.n_wg + 1));
-      L.wg_head.alloc(&c, sizeof(uint32_t) * head.size());
-      L.wg_nodes.alloc(&c, sizeof(uint32_t) * std::max<uint32_t>(nptr[L.n_wg], 1));
-      L.inc_loc.alloc(&c, sizeof(uint32_t) * nek);
-      HIP_OK(hipMemcpyAsync(dptr.ptr, nptr.data(), sizeof(uint32_t) * nptr.size(), hipMemcpyHostToDevice, c.stream));
-      HIP_OK(hipMemcpyAsync(L.wg_head.ptr, head.data(), sizeof(uint32_t) * head.size(), hipMemcpyHostToDevice,
-                            c.stream));
-      hipLaunchKernelGGL(k_wg_nodes<true>, dim3(L.n_wg), dim3(kAsmThreads), 0, c.stream, (int)k,
-                         L.wg_rows.as<uint32_t>(), L.inc_ptr.as<uint32_t>(), L.inc.as<uint32_t>(), M.conn.as<uint32_t>(),
-                         dptr.as<uint32_t>(), L.wg_nodes.as<uint32_t>(), L.inc_loc.as<uint32_t>());
+    const uint32_t n_plan = host[0];
+    // node slots: most meshes need few; a workgroup that needs more is counted, and the plans are made again
+    for(uint32_t ns = 64; !host[1];) {
+      L.plan.alloc(&c, (size_t)n_plan * plan_bytes(ns));
+      hipLaunchKernelGGL(k_plan_fill, dim3(n_plan), dim3(kAsmThreads), 0, c.stream, (uint32_t)N, n_plan, (int)k, list_len,
+                         L.periodic, ns, starts, L.row_ptr.as<uint32_t>(), L.inc_ptr.as<uint32_t>(),
+                         L.inc.as<uint32_t>(), back, conn, M.conn.as<uint32_t>(),
+                         contrib_ptr.as<uint32_t>(), contrib.as<uint16_t>(), L.plan.as<unsigned char>(), inf + 2);
       HIP_OK(hipGetLastError());
-      HIP_OK(hipStreamSynchronize(c.stream));   // dptr and the host vectors go out of scope
-      L.wg_nodes_max = mx;
-      L.staged = true;
+      HIP_OK(hipMemcpyAsync(host, inf, sizeof(host), hipMemcpyDeviceToHost, c.stream));
+      HIP_OK(hipStreamSynchronize(c.stream));
+      if(host[2] <= ns) {
+        L.n_plan = n_plan;
+        L.plan_nodes = ns;
+        L.plan_elems = host[3];
+        L.plan_lists = host[4];
+        break;
+      }
+      L.plan.release();
+      if(host[2] > kPlanNodes) break;
+      ns = (host[2] + 3) / 4 * 4;
     }
   }
   HIP_OK(hipStreamSynchronize(c.stream));

@@ -1,0 +1,91 @@
+"""The block-list assembly of the specialised triangles and tetrahedra at the limits of its plans, against the
+oracle: fans whose centre rows fill a workgroup's 128 block lists exactly, miss them by one (the staged
+reduction then serves the system), or fit easily; single elements; periodic links, where a block sums several
+mesh nodes that hold different states.
+
+Bars: FP64 row-relative 1e-12 as everywhere; FP32 1e-6 of the element matrices plus one rounding per summed
+contribution."""
+import numpy as np
+import pytest
+
+from coolfluid3_amd import cabi, cases, meshgen
+from oracle import pyoracle
+from tests.test_gpu_parity import gpu_case, oracle_system, row_rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = cabi.Context(0)
+    yield c
+    c.close()
+
+
+def case_of(etype, coords, conn, periodic=None, seed=5):
+    rng = np.random.default_rng(seed)
+    N, dim = coords.shape
+    return cases.Case("fan", etype, coords, conn.astype(np.uint32), None, 1e-2, 1e-2, u0=rng.uniform(-1, 1, (N, dim)),
+                      p0=rng.uniform(-1, 1, N), periodic=periodic)
+
+
+def triangle_fan(n):
+    """n triangles around node 0, its local index rotating."""
+    a = 2 * np.pi * np.arange(n) / n
+    coords = np.concatenate([[[0.3, 0.2]], np.stack([0.3 + np.cos(a), 0.2 + np.sin(a)], axis=1)])
+    conn = np.stack([np.zeros(n, int), 1 + np.arange(n), 1 + (np.arange(n) + 1) % n], axis=1)
+    return case_of(cabi.TRIAG2D, coords, np.stack([np.roll(c, i % 3) for i, c in enumerate(conn)]))
+
+
+def tetrahedron_fan(n):
+    """n tetrahedra around the edge of nodes 0 and 1, their local indices changing by even permutations."""
+    a = 2 * np.pi * np.arange(n) / n
+    ring = np.stack([np.cos(a), np.sin(a), np.zeros(n)], axis=1)
+    coords = np.concatenate([[[0, 0, -0.5], [0, 0, 0.5]], ring]) + 0.1
+    conn = np.stack([np.zeros(n, int), 2 + np.arange(n), 2 + (np.arange(n) + 1) % n, np.ones(n, int)], axis=1)
+    even = np.array([[0, 1, 2, 3], [1, 0, 3, 2], [2, 3, 0, 1], [3, 2, 1, 0]])
+    return case_of(cabi.TETRA3D, coords, np.stack([c[even[i % 4]] for i, c in enumerate(conn)]))
+
+
+# triangles: 32 + 96 = 128 lists, 33 + 97 = 130; tetrahedra: 96 + 16 + 16 = 128, 97 + 17 + 17 = 131
+@pytest.mark.parametrize("make,n", [(triangle_fan, 3), (triangle_fan, 95), (triangle_fan, 96), (triangle_fan, 97),
+                                    (tetrahedron_fan, 3), (tetrahedron_fan, 95), (tetrahedron_fan, 96),
+                                    (tetrahedron_fan, 97)])
+def test_fans_at_the_list_limit(ctx, oracle, make, n):
+    print(make.__name__, n, flush=True)
+    case = make(n)
+    neq = case.dim + 1
+    start, _, _, vref, rref = oracle_system(oracle, case, theta=0.7)
+    g = gpu_case(ctx, case, theta=0.7, fp32=True)
+    g.assemble(cabi.FP64)
+    v, r = g.system.values(), g.system.vector(cabi.RHS)
+    assert row_rel_err(v, vref, neq, start) <= 1e-12
+    assert np.abs(r - rref).max() <= 1e-12 * np.abs(rref).max()
+    g.assemble(cabi.FP64)
+    assert np.array_equal(g.system.values(), v) and np.array_equal(g.system.vector(cabi.RHS), r)
+    g.assemble(cabi.FP32)
+    assert row_rel_err(g.system.values_fp32().astype(np.float64), vref, neq, start) <= 1e-6 + n * 2.0 ** -24
+    g.close()
+
+
+@pytest.mark.parametrize("etype,n", [(cabi.TRIAG2D, 2), (cabi.TRIAG2D, 5), (cabi.TETRA3D, 2), (cabi.TETRA3D, 4)])
+def test_periodic_blocks_of_several_nodes(ctx, oracle, etype, n):
+    """Periodic in every direction, with states that differ between the linked nodes; at n = 2 an element
+    can hold two nodes of one block row."""
+    print(etype, n, flush=True)
+    dim = 2 if etype == cabi.TRIAG2D else 3
+    coords, conn = meshgen.rect_tris(n, n) if dim == 2 else meshgen.box_tetras(n, n, n)
+    faces = [(np.flatnonzero(coords[:, d] > 1 - 1e-12), np.flatnonzero(coords[:, d] < 1e-12), -np.eye(dim)[d])
+             for d in range(dim)]
+    case = case_of(etype, coords, conn, periodic=cases.periodic_links(coords, faces))
+    p2m = cases.periodic_p2m(*case.periodic)
+    start, cols, slots = oracle.build_sparsity(p2m[case.conn], int(p2m.max()) + 1)
+    et = pyoracle.TRIAG2D if dim == 2 else pyoracle.TETRA3D
+    ua = oracle.linearize_u(case.u0, case.u0, case.u0, case.u0)
+    vref, rref = oracle.ns_assemble_p2m(et, pyoracle.ns_params(dt=case.dt, theta=0.7), coords, case.conn, p2m, case.u0,
+                                        case.p0, ua, np.full(case.n_nodes, case.nu), start, slots)
+    g = gpu_case(ctx, case, theta=0.7)
+    g.assemble(cabi.FP64)
+    assert np.abs(g.system.values() - vref).max() <= 1e-12 * np.abs(vref).max()
+    assert np.abs(g.system.vector(cabi.RHS) - rref).max() <= 1e-12 * np.abs(rref).max()
+    g.close()
