@@ -1296,11 +1296,11 @@ void assemble(Lss& L, Fields& F, const cf3hip_ns_params& prm)
   check_status(c);
 }
 
-void ns_residual(Lss& L, Fields& F, const cf3hip_ns_params& prm, const double* x, double* r)
+void ns_residual(Lss& L, Fields& F, const cf3hip_ns_params& prm, const double* x, double* r, bool pack)
 {
   if(L.periodic)
     CF3_THROW(CF3HIP_ERR_NOT_IMPLEMENTED, "the matrix-free residual (precision form) takes systems without periodic links");
-  AsmArgs g = make_args(L, F, prm);
+  AsmArgs g = make_args(L, F, prm, pack);
   const Mesh& M = *L.mesh;
   Context& c = *L.ctx;
   if(L.xtilde.bytes < sizeof(double) * L.dofs) L.xtilde.alloc(&c, sizeof(double) * L.dofs);

@@ -274,7 +274,8 @@ void lss_clear_conditions(Lss& L);
 // FP32 values, FP64 vectors and accumulation: y = A32 x
 void lss_spmv_mixed(Lss& L, const double* x, double* y, const double* stop = nullptr);
 // matrix-free FP64 residual r = b' - A' x of the NS system (assembly.hip)
-void ns_residual(Lss& L, Fields& F, const cf3hip_ns_params& prm, const double* x, double* r);
+// pack: refresh the packed node records of F first (false: they are those of an earlier call)
+void ns_residual(Lss& L, Fields& F, const cf3hip_ns_params& prm, const double* x, double* r, bool pack = true);
 void ns_solve(Lss& L, Fields& F, const cf3hip_ns_params& nsp, const cf3hip_solver_params& prm,
               cf3hip_solve_stats& st);
 // stop (optional, device): a Krylov loop's stop flag; the product is skipped once it is set

@@ -16,6 +16,7 @@
 
 #include "arnoldi.hpp"
 #include "internal.hpp"
+#include "lanes.hpp"
 #include "spmv4.hpp"
 
 namespace cf3hip {
@@ -23,6 +24,7 @@ namespace cf3hip {
 namespace {
 
 constexpr int kRT = 256;   // reduction block size
+constexpr unsigned kFusedSpmvBlocks = 2048;   // workgroups of the fused products (8 per CU)
 
 inline unsigned red_grid(uint64_t n) { return std::min<unsigned>(kMaxRedBlocks, grid_for(n, kRT)); }
 
@@ -30,9 +32,9 @@ template<int NDOT>
 __device__ inline void block_reduce_store(double (&v)[NDOT], double* partials, unsigned G)
 {
   __shared__ double sh[NDOT][kRT / 64];
+#pragma unroll
   for(int d = 0; d < NDOT; ++d) {
-    double x = v[d];
-    for(int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off, 64);
+    const double x = lanes::sum64(v[d]);
     if((threadIdx.x & 63) == 0) sh[d][threadIdx.x >> 6] = x;
   }
   __syncthreads();
@@ -62,7 +64,7 @@ __global__ void k_finalize(const double* __restrict__ partials, unsigned G, doub
   for(int d = 0; d < NDOT; ++d) {
     double s = 0.;
     for(unsigned i = threadIdx.x; i < G; i += kRT) s += partials[d * G + i];
-    for(int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
+    s = lanes::sum64(s);
     if((threadIdx.x & 63) == 0) sh[d][threadIdx.x >> 6] = s;
   }
   __syncthreads();
@@ -111,48 +113,105 @@ __global__ void k_finalize(const double* __restrict__ partials, unsigned G, doub
 // iteration parity.
 enum { S_RHO_EVEN = S_RHO, S_RHO_ODD = S_RHO_PREV, S_MAXR_EVEN = S_MAXR };
 
-// sum of G partials per dot product (partials[d * G + i]), result in every thread of the workgroup
-template<int NDOT>
-__device__ inline void workgroup_sum(const double* __restrict__ partials, unsigned G, double (&out)[NDOT])
+// Thread's share of the G <= MAXG partials of NDOT dot products (partials[d * G + i]), in the order of
+// k_finalize.  The loads of all rounds are issued together, ahead of whatever waits for them.
+template<int NDOT, int MAXG>
+__device__ inline void load_partials(const double* __restrict__ partials, unsigned G, double* out)
 {
-  __shared__ double sh[NDOT][kRT / 64];
+  constexpr int U = (MAXG + kRT - 1) / kRT;
+  double v[NDOT][U];
+#pragma unroll
+  for(int d = 0; d < NDOT; ++d)
+#pragma unroll
+    for(int u = 0; u < U; ++u) {
+      v[d][u] = 0.;
+      if((unsigned)(u * kRT) < G) {
+        const unsigned i = threadIdx.x + (unsigned)(u * kRT);
+        const double x = partials[d * G + min(i, G - 1)];
+        v[d][u] = i < G ? x : 0.;
+      }
+    }
+#pragma unroll
   for(int d = 0; d < NDOT; ++d) {
     double s = 0.;
-    for(unsigned i = threadIdx.x; i < G; i += kRT) s += partials[d * G + i];
-    for(int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-    if((threadIdx.x & 63) == 0) sh[d][threadIdx.x >> 6] = s;
-  }
-  __syncthreads();
-  for(int d = 0; d < NDOT; ++d) {
-    double s = 0.;
-    for(int w = 0; w < kRT / 64; ++w) s += sh[d][w];
+#pragma unroll
+    for(int u = 0; u < U; ++u) s += v[d][u];
     out[d] = s;
   }
 }
 
+// sums over the workgroup of N values per thread, result in every thread; `flag` of thread 0 is handed to
+// every thread with them (one barrier)
+template<int N>
+__device__ inline bool workgroup_sum(double (&v)[N], bool flag = false)
+{
+  __shared__ double sh[N][kRT / 64];
+  __shared__ int s_flag;
+#pragma unroll
+  for(int d = 0; d < N; ++d) {
+    const double s = lanes::sum64(v[d]);
+    if((threadIdx.x & 63) == 0) sh[d][threadIdx.x >> 6] = s;
+  }
+  if(threadIdx.x == 0) s_flag = flag ? 1 : 0;
+  __syncthreads();
+#pragma unroll
+  for(int d = 0; d < N; ++d) {
+    double s = 0.;
+    for(int w = 0; w < kRT / 64; ++w) s += sh[d][w];
+    v[d] = s;
+  }
+  return s_flag != 0;
+}
+
 __device__ inline bool leader() { return blockIdx.x == 0 && threadIdx.x == 0; }
+
+// Elements a thread of the vector kernels has in flight.  Its first ones are loaded before the scalars of the
+// iteration are known: on small systems a launch is one chain of load, reduction and update, so every load
+// that can start at once does.  Measured per launch (p / s / x update, us): 16 k rows of one equation
+// 4.5 / 3.9 / 5.1 -> 4.0 / 3.7 / 5.2; 64^3 tetrahedra
+// 14.0 / 13.1 / 21.3 -> 11.6 / 11.0 / 20.4.
+constexpr int kVecU = 4;
+
+template<typename R>
+__device__ __forceinline__ void load_vec(const R* __restrict__ a, uint64_t i, uint64_t stride, uint64_t n, R (&v)[kVecU])
+{
+#pragma unroll
+  for(int u = 0; u < kVecU; ++u)
+    if(u * stride < n) v[u] = a[min(i + u * stride, n - 1)];
+}
 
 // Start of iteration `it`: finalise iteration it-1 from the partials px = (||r||^2, rh . r) -- count,
 // convergence / breakdown test (rel: also the residual-replacement test of the reliable phase) -- then,
 // unless stopped or fin_only, p = r + beta (p - omega v), ph = D^-1 p.
 template<typename R>
-__global__ void k_fb_p(uint64_t n, double* __restrict__ S, int it, int rel, int fin_only, unsigned Gx,
-                       const double* __restrict__ px, const R* __restrict__ r, R* __restrict__ p,
-                       const R* __restrict__ v, R* __restrict__ ph, const R* __restrict__ dinv)
+__global__ __launch_bounds__(kRT) void k_fb_p(uint64_t n, double* __restrict__ S, int it, int rel, int fin_only,
+                                              unsigned Gx, const double* __restrict__ px, const R* __restrict__ r,
+                                              R* __restrict__ p, const R* __restrict__ v, R* __restrict__ ph,
+                                              const R* __restrict__ dinv)
 {
-  // the leader of this launch may raise the stop flag while other workgroups start: read it once per
-  // workgroup, so a workgroup returns or proceeds as a whole (workgroup_sum needs every wave)
-  __shared__ int s_stop;
-  if(threadIdx.x == 0) s_stop = S[S_STOP] != 0. ? 1 : 0;
-  __syncthreads();
-  if(s_stop) return;
-  double red[2];
-  workgroup_sum<2>(px, Gx, red);
-  const double rn2 = red[0], rho = red[1];
-  const bool conv = S[S_SCONV] != 0. || rn2 <= S[S_THR2];
-  bool stop = conv || !isfinite(rn2) || rho == 0. || S[S_OMEGA] == 0.;
+  const uint64_t stride = (uint64_t)gridDim.x * kRT;
+  uint64_t i = (uint64_t)blockIdx.x * kRT + threadIdx.x;
+  R rv[kVecU], pv[kVecU], vv[kVecU], dv[kVecU];
+  auto load = [&] {
+    load_vec(r, i, stride, n, rv);
+    load_vec(p, i, stride, n, pv);
+    load_vec(v, i, stride, n, vv);
+    load_vec(dinv, i, stride, n, dv);
+  };
+  if(!fin_only) load();
+  // the leader of this launch may raise the stop flag while other workgroups start: thread 0's reading
+  // decides for its workgroup, which returns or proceeds as a whole
+  const bool stopped = S[S_STOP] != 0.;
+  const double thr2 = S[S_THR2], sconv = S[S_SCONV], omega_d = S[S_OMEGA], alpha = S[S_ALPHA], delta = S[S_DELTA];
   const double maxr = S[(it & 1) ? S_MAXR_EVEN : S_MAXR_ODD];   // after iteration it - 1
-  if(rel) stop = stop || sqrt(rn2) < S[S_DELTA] * maxr;
+  const double rho_old = S[(it & 1) ? S_RHO_EVEN : S_RHO_ODD];
+  double red[2];
+  load_partials<2, kMaxRedBlocks>(px, Gx, red);
+  if(workgroup_sum<2>(red, stopped)) return;
+  const double rn2 = red[0], rho = red[1];
+  const bool conv = sconv != 0. || rn2 <= thr2;
+  bool stop = conv || !isfinite(rn2) || rho == 0. || omega_d == 0.;
+  if(rel) stop = stop || sqrt(rn2) < delta * maxr;
   if(leader()) {
     S[S_RN2] = rn2;
     S[(it & 1) ? S_RHO_ODD : S_RHO_EVEN] = rho;
@@ -161,14 +220,19 @@ __global__ void k_fb_p(uint64_t n, double* __restrict__ S, int it, int rel, int 
     S[(it & 1) ? S_MAXR_ODD : S_MAXR_EVEN] = (rel && !stop) ? fmax(maxr, sqrt(rn2)) : maxr;
   }
   if(stop || fin_only) return;
-  const double rho_old = S[(it & 1) ? S_RHO_EVEN : S_RHO_ODD];
-  const R beta = (R)((rho / rho_old) * (S[S_ALPHA] / S[S_OMEGA]));
-  const R omega = (R)S[S_OMEGA];
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for(uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    const R pi = r[i] + beta * (p[i] - omega * v[i]);
-    p[i] = pi;
-    ph[i] = dinv[i] * pi;
+  const R beta = (R)((rho / rho_old) * (alpha / omega_d));
+  const R omega = (R)omega_d;
+  for(;;) {
+#pragma unroll
+    for(int u = 0; u < kVecU; ++u)
+      if(i + u * stride < n) {
+        const R pi = rv[u] + beta * (pv[u] - omega * vv[u]);
+        p[i + u * stride] = pi;
+        ph[i + u * stride] = dv[u] * pi;
+      }
+    i += kVecU * stride;
+    if(i >= n) break;
+    load();
   }
 }
 
@@ -182,11 +246,12 @@ __global__ __launch_bounds__(kRT) void k_spmv4_dot(uint32_t N, const uint32_t* _
                                                    const XR* __restrict__ d0, const double* __restrict__ S,
                                                    double* __restrict__ partials)
 {
-  if(S[S_STOP] != 0.) return;
+  const double stop = S[S_STOP];
   double acc[NDOT];
   for(int d = 0; d < NDOT; ++d) acc[d] = 0.;
   const int l = threadIdx.x & 15;
   const uint32_t step = gridDim.x * (kRT / 16);
+  if(stop != 0.) return;
   for(uint32_t row = blockIdx.x * (kRT / 16) + (threadIdx.x >> 4); row < N; row += step) {
     int a;
     bool out;
@@ -229,7 +294,7 @@ __global__ __launch_bounds__(kRT) void k_spmvn_dot(uint32_t N, const uint32_t* _
         for(int j = 0; j < NEQ; ++j) ys[i] += (double)b[i * NEQ + j] * xc[j];
     }
     for(int i = 0; i < NEQ; ++i)
-      for(int off = LANES / 2; off > 0; off >>= 1) ys[i] += __shfl_xor(ys[i], off, LANES);
+      ys[i] = LANES == 8 ? lanes::sum8(ys[i]) : lanes::sum16(ys[i]);
     if(l == 0)
       for(int i = 0; i < NEQ; ++i) {
         const uint64_t o = (uint64_t)row * NEQ + i;
@@ -243,26 +308,44 @@ __global__ __launch_bounds__(kRT) void k_spmvn_dot(uint32_t N, const uint32_t* _
 
 // alpha = rho / (rh . v) from the partials pv; s = r - alpha v, sh = D^-1 s, partials ||s||^2
 template<typename R>
-__global__ void k_fb_s(uint64_t n, double* __restrict__ S, int it, unsigned Gv, const double* __restrict__ pv,
-                       const R* __restrict__ r, const R* __restrict__ v, R* __restrict__ s, R* __restrict__ sh,
-                       const R* __restrict__ dinv, double* __restrict__ ps)
+__global__ __launch_bounds__(kRT) void k_fb_s(uint64_t n, double* __restrict__ S, int it, unsigned Gv,
+                                              const double* __restrict__ pv, const R* __restrict__ r,
+                                              const R* __restrict__ v, R* __restrict__ s, R* __restrict__ sh,
+                                              const R* __restrict__ dinv, double* __restrict__ ps)
 {
-  if(S[S_STOP] != 0.) return;
+  const uint64_t stride = (uint64_t)gridDim.x * kRT;
+  uint64_t i = (uint64_t)blockIdx.x * kRT + threadIdx.x;
+  R rv[kVecU], vv[kVecU], dv[kVecU];
+  auto load = [&] {
+    load_vec(r, i, stride, n, rv);
+    load_vec(v, i, stride, n, vv);
+    load_vec(dinv, i, stride, n, dv);
+  };
+  load();
+  const double stop = S[S_STOP], rho = S[(it & 1) ? S_RHO_ODD : S_RHO_EVEN];
   double red[1];
-  workgroup_sum<1>(pv, Gv, red);
-  const double alpha_d = S[(it & 1) ? S_RHO_ODD : S_RHO_EVEN] / red[0];
+  load_partials<1, kFusedSpmvBlocks>(pv, Gv, red);
+  if(stop != 0.) return;
+  workgroup_sum<1>(red);
+  const double alpha_d = rho / red[0];
   if(leader()) {
     S[S_RHV] = red[0];
     S[S_ALPHA] = alpha_d;
   }
   const R alpha = (R)alpha_d;
   double acc[1] = {0.};
-  const uint64_t stride = (uint64_t)gridDim.x * kRT;
-  for(uint64_t i = (uint64_t)blockIdx.x * kRT + threadIdx.x; i < n; i += stride) {
-    const R si = r[i] - alpha * v[i];
-    s[i] = si;
-    sh[i] = dinv[i] * si;
-    acc[0] += (double)si * (double)si;
+  for(;;) {
+#pragma unroll
+    for(int u = 0; u < kVecU; ++u)
+      if(i + u * stride < n) {
+        const R si = rv[u] - alpha * vv[u];
+        s[i + u * stride] = si;
+        sh[i + u * stride] = dv[u] * si;
+        acc[0] += (double)si * (double)si;
+      }
+    i += kVecU * stride;
+    if(i >= n) break;
+    load();
   }
   block_reduce_store<1>(acc, ps, gridDim.x);
 }
@@ -270,34 +353,274 @@ __global__ void k_fb_s(uint64_t n, double* __restrict__ S, int it, unsigned Gv, 
 // omega = (t . s) / (t . t) (0 once ||s|| meets the tolerance) from the partials ps, pt;
 // x += alpha ph + omega sh, r = s - omega t, partials (||r||^2, rh . r)
 template<typename R>
-__global__ void k_fb_x(uint64_t n, double* __restrict__ S, unsigned Gs, const double* __restrict__ ps, unsigned Gt,
-                       const double* __restrict__ pt, R* __restrict__ x, const R* __restrict__ ph,
-                       const R* __restrict__ sh, R* __restrict__ r, const R* __restrict__ s, const R* __restrict__ t,
-                       const R* __restrict__ rh, double* __restrict__ px)
+__global__ __launch_bounds__(kRT) void k_fb_x(uint64_t n, double* __restrict__ S, unsigned Gs,
+                                              const double* __restrict__ ps, unsigned Gt, const double* __restrict__ pt,
+                                              R* __restrict__ x, const R* __restrict__ ph, const R* __restrict__ sh,
+                                              R* __restrict__ r, const R* __restrict__ s, const R* __restrict__ t,
+                                              const R* __restrict__ rh, double* __restrict__ px)
 {
-  if(S[S_STOP] != 0.) return;
-  double rs[1], rt[2];
-  workgroup_sum<1>(ps, Gs, rs);
-  __syncthreads();
-  workgroup_sum<2>(pt, Gt, rt);
-  const bool sconv = rs[0] <= S[S_THR2];
-  const double omega_d = sconv ? 0. : rt[0] / rt[1];
+  const uint64_t stride = (uint64_t)gridDim.x * kRT;
+  uint64_t i = (uint64_t)blockIdx.x * kRT + threadIdx.x;
+  R xv[kVecU], pv[kVecU], hv[kVecU], sv[kVecU], tv[kVecU], rv[kVecU];
+  auto load = [&] {
+    load_vec(x, i, stride, n, xv);
+    load_vec(ph, i, stride, n, pv);
+    load_vec(sh, i, stride, n, hv);
+    load_vec(s, i, stride, n, sv);
+    load_vec(t, i, stride, n, tv);
+    load_vec(rh, i, stride, n, rv);
+  };
+  load();
+  const double stop = S[S_STOP], thr2 = S[S_THR2], alpha_d = S[S_ALPHA];
+  double red[3];   // ||s||^2, t . s, t . t
+  load_partials<1, kMaxRedBlocks>(ps, Gs, red);
+  load_partials<2, kFusedSpmvBlocks>(pt, Gt, red + 1);
+  if(stop != 0.) return;
+  workgroup_sum<3>(red);
+  const bool sconv = red[0] <= thr2;
+  const double omega_d = sconv ? 0. : red[1] / red[2];
   if(leader()) {
-    S[S_SN2] = rs[0];
+    S[S_SN2] = red[0];
     S[S_SCONV] = sconv ? 1. : 0.;
-    S[S_TS] = rt[0];
-    S[S_TT] = rt[1];
+    S[S_TS] = red[1];
+    S[S_TT] = red[2];
     S[S_OMEGA] = omega_d;
   }
-  const R alpha = (R)S[S_ALPHA], omega = (R)omega_d;
+  const R alpha = (R)alpha_d, omega = (R)omega_d;
   double acc[2] = {0., 0.};
+  for(;;) {
+#pragma unroll
+    for(int u = 0; u < kVecU; ++u)
+      if(i + u * stride < n) {
+        x[i + u * stride] = xv[u] + (alpha * pv[u] + omega * hv[u]);
+        const R ri = sv[u] - omega * tv[u];
+        r[i + u * stride] = ri;
+        acc[0] += (double)ri * (double)ri;
+        acc[1] += (double)rv[u] * (double)ri;
+      }
+    i += kVecU * stride;
+    if(i >= n) break;
+    load();
+  }
+  block_reduce_store<2>(acc, px, gridDim.x);
+}
+
+// ---- three-launch iteration for small systems (FP64 vectors, neq = 1 to 4) ----
+// There a launch costs its latency (4 to 5 us) and not its bytes, so the p and s updates move into the
+// products: the product kernel forms the entries of D^-1 p (D^-1 s) it needs from r, p, v and D^-1 as it
+// gathers them, every entry by the arithmetic of k_fb_p (k_fb_s), and the row's owner stores p.  What a
+// gather reads no workgroup of the launch writes: p and v alternate between two buffers by iteration parity.
+// k_fb_x's work then starts from r, v and p.  fused_gather_blocks says where the extra gathers stop paying.
+//   STAGE 1: p' = r + beta (p - omega v), y = A D^-1 p', partials rh . y
+//   STAGE 2: s = r - alpha v,             y = A D^-1 s,  partials s . s, y . s, y . y
+template<typename VR, int NEQ, int STAGE>
+__global__ __launch_bounds__(kRT) void k_fb_product(uint32_t N, const uint32_t* __restrict__ row_ptr,
+                                                    const uint32_t* __restrict__ cols, const VR* __restrict__ vals,
+                                                    double* __restrict__ S, int it, int rel, unsigned G,
+                                                    const double* __restrict__ part, const double* __restrict__ r,
+                                                    const double* __restrict__ p, const double* __restrict__ v,
+                                                    const double* __restrict__ dinv, const double* __restrict__ rh,
+                                                    double* __restrict__ pnew, double* __restrict__ y,
+                                                    double* __restrict__ out)
+{
+  // lanes per node row; neq = 4: 8 lanes per block, a lane takes two columns of one block row, 4 blocks per
+  // trip and half; otherwise a lane takes whole blocks
+  constexpr int LANES = NEQ == 1 ? 8 : 16;
+  constexpr bool WIDE = NEQ == 4;
+  constexpr int BL = WIDE ? 2 : LANES;             // blocks of a row side by side
+  constexpr int T = 2;                             // blocks per lane and trip
+  constexpr int CW = WIDE ? 2 : NEQ, RW = WIDE ? 1 : NEQ;
+  const uint32_t l = threadIdx.x & (LANES - 1);
+  const uint32_t sub = WIDE ? l >> 3 : l, c0 = WIDE ? 2 * (l & 1) : 0, a0 = WIDE ? (l & 7) >> 1 : 0;
+  const bool own = WIDE ? (l < 8 && (l & 1) == 0) : l == 0;
+  const uint32_t step = gridDim.x * (kRT / LANES);
+  uint32_t row = blockIdx.x * (kRT / LANES) + threadIdx.x / LANES;
+
+  uint32_t q = 0, q1 = 0;
+  double m[T][RW][CW], gr[T][CW], gp[T][CW], gv[T][CW], gd[T][CW];
+  double wr[RW], wp[RW], wv[RW], wh[RW];           // the owner's entries of its row
+  auto row_begin = [&] {
+    q = q1 = 0;
+    if(row >= N) return;
+    q = row_ptr[row] + sub;
+    q1 = row_ptr[row + 1];
+    if(own)
+#pragma unroll
+      for(int i = 0; i < RW; ++i) {
+        const uint64_t o = (uint64_t)row * NEQ + a0 + i;
+        wr[i] = r[o];
+        wv[i] = v[o];
+        if constexpr(STAGE == 1) { wp[i] = p[o]; wh[i] = rh[o]; }
+      }
+  };
+  auto load = [&] {
+#pragma unroll
+    for(int k = 0; k < T; ++k) {
+      const uint32_t qq = min(q + (uint32_t)(BL * k), q1 - 1);
+      const VR* b = vals + (uint64_t)qq * NEQ * NEQ + a0 * NEQ + c0;
+      const uint64_t o = (uint64_t)cols[qq] * NEQ + c0;
+#pragma unroll
+      for(int i = 0; i < RW; ++i)
+#pragma unroll
+        for(int j = 0; j < CW; ++j) m[k][i][j] = (double)b[i * NEQ + j];
+#pragma unroll
+      for(int j = 0; j < CW; ++j) {
+        gr[k][j] = r[o + j];
+        gv[k][j] = v[o + j];
+        gd[k][j] = dinv[o + j];
+        if constexpr(STAGE == 1) gp[k][j] = p[o + j];
+      }
+    }
+  };
+  row_begin();
+  if(q < q1) load();
+
+  // the scalars of the iteration, as in k_fb_p and k_fb_s
+  const bool stopped = S[S_STOP] != 0.;
+  double c_b, c_o = 0.;   // STAGE 1: beta, omega; STAGE 2: alpha
+  if constexpr(STAGE == 1) {
+    const double thr2 = S[S_THR2], sconv = S[S_SCONV], omega = S[S_OMEGA], alpha = S[S_ALPHA], delta = S[S_DELTA];
+    const double maxr = S[(it & 1) ? S_MAXR_EVEN : S_MAXR_ODD];
+    const double rho_old = S[(it & 1) ? S_RHO_EVEN : S_RHO_ODD];
+    double red[2];
+    load_partials<2, kMaxRedBlocks>(part, G, red);
+    if(workgroup_sum<2>(red, stopped)) return;
+    const double rn2 = red[0], rho = red[1];
+    bool stop = sconv != 0. || rn2 <= thr2 || !isfinite(rn2) || rho == 0. || omega == 0.;
+    if(rel) stop = stop || sqrt(rn2) < delta * maxr;
+    if(leader()) {
+      S[S_RN2] = rn2;
+      S[(it & 1) ? S_RHO_ODD : S_RHO_EVEN] = rho;
+      S[S_ITER] = (double)it;
+      if(stop) S[S_STOP] = 1.;
+      S[(it & 1) ? S_MAXR_ODD : S_MAXR_EVEN] = (rel && !stop) ? fmax(maxr, sqrt(rn2)) : maxr;
+    }
+    if(stop) return;
+    c_b = (rho / rho_old) * (alpha / omega);
+    c_o = omega;
+  } else {
+    const double rho = S[(it & 1) ? S_RHO_ODD : S_RHO_EVEN];
+    double red[1];
+    load_partials<1, kFusedSpmvBlocks>(part, G, red);
+    if(stopped) return;
+    workgroup_sum<1>(red);
+    c_b = rho / red[0];
+    if(leader()) {
+      S[S_RHV] = red[0];
+      S[S_ALPHA] = c_b;
+    }
+  }
+  auto update = [&](double rr, double pp, double vv) {
+    if constexpr(STAGE == 1) return rr + c_b * (pp - c_o * vv);
+    else return rr - c_b * vv;
+  };
+  constexpr int ND = STAGE == 1 ? 1 : 3;
+  double acc[ND];
+#pragma unroll
+  for(int d = 0; d < ND; ++d) acc[d] = 0.;
+  while(row < N) {
+    double ys[RW];
+#pragma unroll
+    for(int i = 0; i < RW; ++i) ys[i] = 0.;
+    while(q < q1) {
+#pragma unroll
+      for(int k = 0; k < T; ++k) {
+        double x[CW];
+#pragma unroll
+        for(int j = 0; j < CW; ++j) x[j] = gd[k][j] * update(gr[k][j], STAGE == 1 ? gp[k][j] : 0., gv[k][j]);
+#pragma unroll
+        for(int i = 0; i < RW; ++i) {
+          double sum = m[k][i][0] * x[0];
+#pragma unroll
+          for(int j = 1; j < CW; ++j) sum += m[k][i][j] * x[j];
+          ys[i] = q + BL * k < q1 ? ys[i] + sum : ys[i];
+        }
+      }
+      q += BL * T;
+      if(q < q1) load();
+    }
+#pragma unroll
+    for(int i = 0; i < RW; ++i) {
+      if constexpr(WIDE) {
+        ys[i] += lanes::move<lanes::kXor1>(ys[i]);
+        ys[i] += lanes::move<lanes::kNext8>(ys[i]);
+      } else {
+        ys[i] = LANES == 8 ? lanes::sum8(ys[i]) : lanes::sum16(ys[i]);
+      }
+    }
+    if(own)
+#pragma unroll
+      for(int i = 0; i < RW; ++i) {
+        const uint64_t o = (uint64_t)row * NEQ + a0 + i;
+        const double u = update(wr[i], STAGE == 1 ? wp[i] : 0., wv[i]);
+        y[o] = ys[i];
+        if constexpr(STAGE == 1) {
+          pnew[o] = u;
+          acc[0] += wh[i] * ys[i];
+        } else {
+          acc[0] += u * u;
+          acc[ND > 1 ? 1 : 0] += ys[i] * u;
+          acc[ND > 2 ? 2 : 0] += ys[i] * ys[i];
+        }
+      }
+    row += step;
+    row_begin();
+    if(q < q1) load();
+  }
+  block_reduce_store<ND>(acc, out, gridDim.x);
+}
+
+// omega from the partials pt = (s . s, t . s, t . t); x += alpha D^-1 p + omega D^-1 s, r = s - omega t with
+// s = r - alpha v; partials (||r||^2, rh . r)
+__global__ __launch_bounds__(kRT) void k_fb_update(uint64_t n, double* __restrict__ S, unsigned Gt,
+                                                   const double* __restrict__ pt, double* __restrict__ x,
+                                                   const double* __restrict__ p, const double* __restrict__ v,
+                                                   const double* __restrict__ t, const double* __restrict__ dinv,
+                                                   double* __restrict__ r, const double* __restrict__ rh,
+                                                   double* __restrict__ px)
+{
   const uint64_t stride = (uint64_t)gridDim.x * kRT;
-  for(uint64_t i = (uint64_t)blockIdx.x * kRT + threadIdx.x; i < n; i += stride) {
-    x[i] += alpha * ph[i] + omega * sh[i];
-    const R ri = s[i] - omega * t[i];
-    r[i] = ri;
-    acc[0] += (double)ri * (double)ri;
-    acc[1] += (double)rh[i] * (double)ri;
+  uint64_t i = (uint64_t)blockIdx.x * kRT + threadIdx.x;
+  double xv[kVecU], pv[kVecU], vv[kVecU], tv[kVecU], dv[kVecU], rv[kVecU], hv[kVecU];
+  auto load = [&] {
+    load_vec(x, i, stride, n, xv);
+    load_vec(p, i, stride, n, pv);
+    load_vec(v, i, stride, n, vv);
+    load_vec(t, i, stride, n, tv);
+    load_vec(dinv, i, stride, n, dv);
+    load_vec((const double*)r, i, stride, n, rv);
+    load_vec(rh, i, stride, n, hv);
+  };
+  load();
+  const double stop = S[S_STOP], thr2 = S[S_THR2], alpha = S[S_ALPHA];
+  double red[3];
+  load_partials<3, kFusedSpmvBlocks>(pt, Gt, red);
+  if(stop != 0.) return;
+  workgroup_sum<3>(red);
+  const bool sconv = red[0] <= thr2;
+  const double omega = sconv ? 0. : red[1] / red[2];
+  if(leader()) {
+    S[S_SN2] = red[0];
+    S[S_SCONV] = sconv ? 1. : 0.;
+    S[S_TS] = red[1];
+    S[S_TT] = red[2];
+    S[S_OMEGA] = omega;
+  }
+  double acc[2] = {0., 0.};
+  for(;;) {
+#pragma unroll
+    for(int u = 0; u < kVecU; ++u)
+      if(i + u * stride < n) {
+        const double si = rv[u] - alpha * vv[u];
+        x[i + u * stride] = xv[u] + (alpha * (dv[u] * pv[u]) + omega * (dv[u] * si));
+        const double ri = si - omega * tv[u];
+        r[i + u * stride] = ri;
+        acc[0] += ri * ri;
+        acc[1] += hv[u] * ri;
+      }
+    i += kVecU * stride;
+    if(i >= n) break;
+    load();
   }
   block_reduce_store<2>(acc, px, gridDim.x);
 }
@@ -404,10 +727,21 @@ __global__ void k_set_scalars(double* S, double thr2, int it0)
   S[S_STOP] = 0.; S[S_ITER] = (double)it0;
 }
 
+// residual replacement: the recurrence goes on with residual norm maxr
+__global__ void k_reseed(double* S, double maxr)
+{
+  S[S_SCONV] = 0.; S[S_STOP] = 0.; S[S_MAXR] = maxr; S[S_MAXR_ODD] = maxr;
+}
+
+constexpr int kFirstBatch = 4;
 constexpr int kMaxBatch = 16;   // iterations enqueued between two host reads of the scalars
-constexpr unsigned kFusedSpmvBlocks = 2048;   // workgroups of the fused products (8 per CU)
 // partials of the fused iteration: (||r||^2, rh . r), rh . v, ||s||^2, (t . s, t . t)
-constexpr size_t kFusedPartials = 2 * kMaxRedBlocks + kFusedSpmvBlocks + kMaxRedBlocks + 2 * kFusedSpmvBlocks;
+constexpr size_t kFusedPartials = 2 * kMaxRedBlocks + kFusedSpmvBlocks + kMaxRedBlocks + 3 * kFusedSpmvBlocks;
+// Node blocks up to which an iteration takes three launches, by equations per node.  Measured per iteration, five
+// -> three launches (us): 4 equations 16^3 cells 30 -> 24, 24^3 (218 k blocks) 34 -> 33, 28^3 43 -> 51; 1 equation
+// (a semi-implicit step, ms) 128^2 17.2 -> 11.7, 200^2 (360 k) 25.8 -> 25.0, 256^2 39.6 -> 40.0; 3 equations
+// 64^2 (29 k) 21.3 -> 19.8, 128^2 25 -> 35.  2 equations: between their neighbours.
+inline uint64_t fused_gather_blocks(int neq) { return neq == 1 ? 360000 : neq == 2 ? 120000 : neq == 3 ? 40000 : 220000; }
 
 template<typename Src, typename Dst>
 __global__ void k_convert_scaled(uint64_t n, const Src* __restrict__ a, Dst* __restrict__ b, double scale)
@@ -461,7 +795,7 @@ struct Recurrence {
   R *x, *r, *rh, *p, *v, *ph, *s, *sh, *t;
   const R* dinv;
   int rel;
-  bool fused;
+  bool fused, gather;
   unsigned Gv, Gs;
   double *part, *px, *pv, *ps, *pt;
   int next = 0;   // index of the next iteration to enqueue
@@ -477,6 +811,7 @@ struct Recurrence {
     // rows per workgroup of the fused products: 16 lanes per node row, 8 for scalar rows (k_spmvn_dot)
     Gs = std::min<unsigned>(kFusedSpmvBlocks, grid_for(L.n_nodes, kRT / (L.neq == 1 ? 8 : 16)));
     part = c.red_partials.as<double>();
+    gather = fused && sizeof(R) == sizeof(double) && L.n_blocks <= fused_gather_blocks(L.neq);
     if(fused) {
       if(!c.fused_partials.ptr) c.fused_partials.alloc(&c, sizeof(double) * kFusedPartials);
       px = c.fused_partials.as<double>();
@@ -491,28 +826,45 @@ struct Recurrence {
     return fused ? sc.v[(it & 1) ? S_RHO_ODD : S_RHO_EVEN] : sc.v[S_RHO];
   }
 
-  // r holds a new residual.  restart: fresh recurrence from iteration it0 (rh = r, p = v = 0, scalars
-  // reset); otherwise a residual replacement that keeps the search directions and scalars.
-  void seed(double thr2, bool restart, int it0)
+  // p and v at the start of iteration it: in the three-launch form they alternate with the vectors that form
+  // does not store (D^-1 p and s)
+  R* cur_p(int it) const { return gather && (it & 1) ? ph : p; }
+  R* cur_v(int it) const { return gather && (it & 1) ? s : v; }
+
+  // r holds a new residual of norm rnorm.  restart: fresh recurrence from iteration it0 (rh = r, p = v = 0,
+  // scalars reset); otherwise a residual replacement that keeps the search directions and scalars.  dots: the
+  // partials (||r||^2, rh . r) are there already (residual_norm).
+  void seed(double thr2, bool restart, int it0, double rnorm, bool dots = false)
   {
     if(restart) {
       if(rh != r) HIP_OK(hipMemcpyAsync(rh, r, sizeof(R) * n, hipMemcpyDeviceToDevice, c.stream));
-      fill(p, 0.);
-      fill(v, 0.);
+      fill(cur_p(it0), 0.);
+      fill(cur_v(it0), 0.);
       hipLaunchKernelGGL(k_set_scalars, dim3(1), dim3(1), 0, c.stream, S, thr2, it0);
-    } else {
-      hipLaunchKernelGGL(k_set_scalar, dim3(1), dim3(1), 0, c.stream, S, (int)S_SCONV, 0.);
-      hipLaunchKernelGGL(k_set_scalar, dim3(1), dim3(1), 0, c.stream, S, (int)S_STOP, 0.);
     }
-    if(fused) {
-      hipLaunchKernelGGL(k_dot2<R>, dim3(Gv), dim3(kRT), 0, c.stream, n, r, r, rh, r, px, (const double*)nullptr);
-    } else {
-      hipLaunchKernelGGL(k_dot2<R>, dim3(Gv), dim3(kRT), 0, c.stream, n, rh, r, (const R*)nullptr, (const R*)nullptr,
-                         part, (const double*)nullptr);
-      hipLaunchKernelGGL(k_finalize<1>, dim3(1), dim3(kRT), 0, c.stream, part, Gv, S, (int)S_RHO, (int)FIN_STORE);
+    if(!restart || rel) hipLaunchKernelGGL(k_reseed, dim3(1), dim3(1), 0, c.stream, S, rnorm);
+    if(restart || !dots) {
+      if(fused) {
+        hipLaunchKernelGGL(k_dot2<R>, dim3(Gv), dim3(kRT), 0, c.stream, n, r, r, rh, r, px, (const double*)nullptr);
+      } else {
+        hipLaunchKernelGGL(k_dot2<R>, dim3(Gv), dim3(kRT), 0, c.stream, n, rh, r, (const R*)nullptr, (const R*)nullptr,
+                           part, (const double*)nullptr);
+        hipLaunchKernelGGL(k_finalize<1>, dim3(1), dim3(kRT), 0, c.stream, part, Gv, S, (int)S_RHO, (int)FIN_STORE);
+      }
     }
     HIP_OK(hipGetLastError());
     next = it0;
+  }
+
+  // ||r||, with the partials that a following seed needs (fused iteration)
+  double residual_norm()
+  {
+    hipLaunchKernelGGL(k_dot2<R>, dim3(Gv), dim3(kRT), 0, c.stream, n, r, r, rh, r, px, (const double*)nullptr);
+    hipLaunchKernelGGL(k_finalize<2>, dim3(1), dim3(kRT), 0, c.stream, px, Gv, S, (int)S_TMP0, (int)FIN_STORE);
+    HIP_OK(hipGetLastError());
+    Scalars sc;
+    read_scalars(c, sc);
+    return std::sqrt(sc.v[S_TMP0]);
   }
 
   // fused product y = A x with its partial dot products (see k_spmv4_dot / k_spmvn_dot)
@@ -537,6 +889,28 @@ struct Recurrence {
     }
   }
 
+  // one product of the three-launch iteration
+  template<int STAGE>
+  void product(const double* partials, unsigned G, double* y, double* out)
+  {
+    if constexpr(sizeof(R) == sizeof(double)) {
+      const uint32_t* rp = L.row_ptr.as<uint32_t>();
+      const uint32_t* cl = L.cols.as<uint32_t>();
+      // STAGE 1 reads the p and v of this iteration's start and writes the next; STAGE 2 reads the new v
+      double *pn = cur_p(next + 1), *vo = STAGE == 1 ? cur_v(next) : cur_v(next + 1);
+      auto go = [&](auto neq) {
+        hipLaunchKernelGGL((k_fb_product<VR, decltype(neq)::value, STAGE>), dim3(Gs), dim3(kRT), 0, c.stream, L.n_nodes, rp,
+                           cl, vals(), S, next, rel, G, partials, r, cur_p(next), vo, dinv, rh, pn, y, out);
+      };
+      switch(L.neq) {
+        case 4: go(std::integral_constant<int, 4>()); break;
+        case 3: go(std::integral_constant<int, 3>()); break;
+        case 2: go(std::integral_constant<int, 2>()); break;
+        default: go(std::integral_constant<int, 1>()); break;
+      }
+    }
+  }
+
   // nb iterations; afterwards S holds the iteration count, the stop flag and the last residual norm
   void enqueue(int nb)
   {
@@ -544,7 +918,14 @@ struct Recurrence {
       const VR* vl = vals();
       const uint32_t* rp = L.row_ptr.as<uint32_t>();
       const uint32_t* cl = L.cols.as<uint32_t>();
-      for(int k = 0; k < nb; ++k, ++next) {
+      if constexpr(sizeof(R) == sizeof(double))
+        for(int k = 0; gather && k < nb; ++k, ++next) {
+          product<1>(px, Gv, cur_v(next + 1), pv);
+          product<2>(pv, Gs, t, pt);
+          hipLaunchKernelGGL(k_fb_update, dim3(Gv), dim3(kRT), 0, c.stream, n, S, Gs, pt, x, cur_p(next + 1),
+                             cur_v(next + 1), t, dinv, r, rh, px);
+        }
+      for(int k = 0; !gather && k < nb; ++k, ++next) {
         hipLaunchKernelGGL(k_fb_p<R>, dim3(Gv), dim3(kRT), 0, c.stream, n, S, next, rel, 0, Gv, px, r, p, v, ph, dinv);
         spmv_dot<1>(rp, cl, vl, ph, v, rh, pv);
         hipLaunchKernelGGL(k_fb_s<R>, dim3(Gv), dim3(kRT), 0, c.stream, n, S, next, Gs, pv, r, v, s, sh, dinv, ps);
@@ -605,9 +986,9 @@ int bicgstab(Lss& L, const R* b, R* x, R* work, double tol, int maxit, bool& con
   double bn2 = sc.v[S_RN2 + 1];
   if(bn2 == 0.) bn2 = 1.;
   const double thr2 = tol * tol * bn2;
-  rc.seed(thr2, true, 0);
+  rc.seed(thr2, true, 0, 0.);
   conv = sc.v[S_RN2] <= thr2;
-  int it = 0, batch = 1;
+  int it = 0, batch = kFirstBatch;
   while(!conv && it < maxit) {
     rc.enqueue(std::min(batch, maxit - it));
     read_scalars(c, sc);
@@ -1028,30 +1409,29 @@ void reliable_core(Lss& L, Resid resid, const cf3hip_solver_params& prm, cf3hip_
   to_r();
   hipLaunchKernelGGL((k_jacobi<R, float>), dim3(grid_for(n, 256)), dim3(256), 0, c.stream, L.n_nodes, L.neq,
                      L.diag_blk.as<uint32_t>(), L.values32.as<float>(), const_cast<R*>(rc.dinv));
-  rc.seed(thr2, true, 0);
+  hipLaunchKernelGGL(k_set_scalar, dim3(1), dim3(1), 0, c.stream, S, (int)S_DELTA, delta);
+  rc.seed(thr2, true, 0, rtrue);
   bool conv = rtrue * rtrue <= thr2;
   // the fallback is for operators the FP32 recurrence cannot follow: on the 128^3 channel (block-scaled
   // FP32 operator) segments that fail to halve the true residual come in long runs and still converge
   // sooner than the FGMRES phase would, so only a long stall or a true divergence switches
   constexpr int kSwitchStall = 40;
   constexpr double kDiverge = 1e3;
-  // iterations enqueued after a replacement before the first host read (a segment is ~10-40 iterations;
-  // launches past a stop return at once)
-  constexpr int kBatchAfterReplace = 4;
   double rprog = rtrue, rbest = rtrue;
   int stall = 0;
   bool switched = false;
-  hipLaunchKernelGGL(k_set_scalar, dim3(1), dim3(1), 0, c.stream, S, (int)S_MAXR, rtrue);
-  hipLaunchKernelGGL(k_set_scalar, dim3(1), dim3(1), 0, c.stream, S, (int)S_MAXR_ODD, rtrue);
-  hipLaunchKernelGGL(k_set_scalar, dim3(1), dim3(1), 0, c.stream, S, (int)S_DELTA, delta);
-  int it = 0, batch = 1;
+  // Iterations enqueued before a host read: a segment between replacements is about as long as the one
+  // before it, and launches past its stop return at once (about 5 us an iteration, a host read 12), so the
+  // first batch of a segment has the length of the last one, the next ones a few iterations
+  constexpr int kExtraBatch = 3;
+  int it = 0, last = 0, batch = kFirstBatch, segment = 0;
   Scalars sc;
   while(!conv && it < prm.max_iter) {
     rc.enqueue(std::min(batch, prm.max_iter - it));
     read_scalars(c, sc);
     it = (int)sc.v[S_ITER];
     if(sc.v[S_STOP] == 0.) {
-      batch = std::min(2 * batch, kMaxBatch);
+      batch = segment == 0 ? std::min(2 * batch, kMaxBatch) : kExtraBatch;
       continue;
     }
     // reliable update: move the increment into the FP64 solution, replace the residual
@@ -1059,7 +1439,8 @@ void reliable_core(Lss& L, Resid resid, const cf3hip_solver_params& prm, cf3hip_
     flush_increment(L, bs, xhi, xlo);
     resid(xhi, rt);
     ++updates;
-    rtrue = norm2(c, rt, n);
+    constexpr bool joined = !f32;   // the FP64 residual is the recurrence's own: one pass gives both products
+    rtrue = joined && rc.fused ? rc.residual_norm() : norm2(c, rt, n);
     if(rtrue * rtrue <= thr2) { conv = true; break; }
     if(rtrue < 0.5 * rprog) {
       rprog = rtrue;
@@ -1071,11 +1452,10 @@ void reliable_core(Lss& L, Resid resid, const cf3hip_solver_params& prm, cf3hip_
     if(!std::isfinite(rtrue) || rtrue > kDiverge * rbest || stall >= kSwitchStall) { switched = true; break; }
     to_r();
     // breakdown: restart the recurrences from the true residual; otherwise keep the directions
-    rc.seed(thr2, breakdown, it);
-    hipLaunchKernelGGL(k_set_scalar, dim3(1), dim3(1), 0, c.stream, S, (int)S_MAXR, rtrue);
-    hipLaunchKernelGGL(k_set_scalar, dim3(1), dim3(1), 0, c.stream, S, (int)S_MAXR_ODD, rtrue);
-    HIP_OK(hipGetLastError());
-    batch = kBatchAfterReplace;
+    rc.seed(thr2, breakdown, it, rtrue, joined && rc.fused);
+    batch = std::min(std::max(it - last, 2), kMaxBatch);
+    segment = 1;
+    last = it;
   }
   const int spmvs = 2 * it;
   if(switched) {
@@ -1127,7 +1507,12 @@ void ns_solve(Lss& L, Fields& F, const cf3hip_ns_params& nsp, const cf3hip_solve
     CF3_THROW(CF3HIP_ERR_NOT_IMPLEMENTED, "the matrix-free residual models the conditions of the block (VBR) builder; "
                                           "solve the stored CRS system instead");
   // the true residual is evaluated matrix-free from the FP64 element matrices of the fields
-  reliable_bicgstab(L, [&](const double* x, double* r) { ns_residual(L, F, nsp, x, r); }, prm, st);
+  // (their packed node records are the same for the whole solve)
+  bool pack = true;
+  reliable_bicgstab(L, [&](const double* x, double* r) {
+    ns_residual(L, F, nsp, x, r, pack);
+    pack = false;
+  }, prm, st);
 }
 
 // precision form on a stored system: the true residual uses the stored FP64 values and rhs

@@ -6,6 +6,8 @@
 
 #include <cstdint>
 
+#include "lanes.hpp"
+
 namespace cf3hip {
 namespace spmv4 {
 
@@ -40,8 +42,8 @@ __device__ __forceinline__ double row_f64(const uint32_t* __restrict__ row_ptr, 
       acc = q + 2u * k < q1 ? acc + s : acc;
     }
   }
-  acc += __shfl_xor(acc, 1, 16);
-  acc += __shfl_xor(acc, 8, 16);
+  acc += lanes::move<lanes::kXor1>(acc);
+  acc += lanes::move<lanes::kNext8>(acc);
   a = li >> 1;
   out = l < 8 && (l & 1) == 0;
   return acc;
@@ -75,8 +77,8 @@ __device__ __forceinline__ double row_mixed(const uint32_t* __restrict__ row_ptr
       acc = q + 4u * k < q1 ? acc + s : acc;
     }
   }
-  acc += __shfl_xor(acc, 4, 16);
-  acc += __shfl_xor(acc, 8, 16);
+  acc += lanes::move<lanes::kNext4>(acc);
+  acc += lanes::move<lanes::kNext8>(acc);
   out = l < 4;
   return acc;
 }
@@ -105,8 +107,8 @@ __device__ __forceinline__ float row_f32(const uint32_t* __restrict__ row_ptr, c
       acc = q + 4u * k < q1 ? acc + s : acc;
     }
   }
-  acc += __shfl_xor(acc, 4, 16);
-  acc += __shfl_xor(acc, 8, 16);
+  acc += lanes::move<lanes::kNext4>(acc);
+  acc += lanes::move<lanes::kNext8>(acc);
   out = l < 4;
   return acc;
 }
