@@ -1317,7 +1317,7 @@ void ns_residual(Lss& L, Fields& F, const cf3hip_ns_params& prm, const double* x
   else launch_residual<GenericP1<2> >(g, L);
   if(L.bc_n)
     hipLaunchKernelGGL(k_bc_residual, dim3(grid_for(L.bc_n, 256)), dim3(256), 0, c.stream, L.bc_n,
-                       L.bc_dof.as<uint32_t>(), L.bc_vlast.as<double>(), x, r);
+                       L.bc_dof, L.bc_vlast, x, r);
   HIP_OK(hipGetLastError());
 }
 
@@ -1349,9 +1349,7 @@ void batch_assemble(Batch& B, uint32_t n, Lss* const* L, Fields* const* F, const
     if((uint64_t)wg + Li.n_plan > 0xffffffffull || (uint64_t)nodes + Li.n_nodes > 0xffffffffull)
       CF3_THROW(CF3HIP_ERR_LIMIT, "batch too large");
     // ZeroLSS: forget the conditions of the previous step (mask cleared on the batch stream)
-    Li.bc_host.clear();
-    Li.bc_order.clear();
-    Li.bc_n = 0;
+    lss_forget_conditions(Li);
     HIP_OK(hipStreamSynchronize(Li.ctx->stream));
     if(Li.bc_mask.ptr) HIP_OK(hipMemsetAsync(Li.bc_mask.ptr, 0, Li.n_nodes, B.stream));
     HIP_OK(hipMemsetAsync(Li.ctx->status_flag(), 0, sizeof(int), B.stream));   // element-validity flag

@@ -165,11 +165,16 @@ struct Lss {
   uint32_t plan_elems = 0, plan_lists = 0;   // most elements and block lists of a workgroup
   // Dirichlet conditions applied since the last reset (needed by the matrix-free FP64 residual):
   // per dof the first value (column elimination) and the last value (row / solution)
-  std::unordered_map<uint64_t, std::pair<double, double> > bc_host;
-  std::vector<uint64_t> bc_order;
+  // (condition i, in order of first application: its dof, first and last value; bc_slot: condition + 1 of a dof)
+  std::vector<uint32_t> bc_slot;   // dofs entries, made by the first condition of the system
+  std::vector<uint32_t> bc_order;
+  std::vector<double> bc_first, bc_last;
+  std::vector<uint64_t> bc_call;   // per condition the call that applied it last
+  uint64_t bc_calls = 0;
   uint32_t bc_n = 0;
-  DevBuf bc_dof;        // uint32 bc_n
-  DevBuf bc_vlast;      // double bc_n
+  DevBuf bc_upload;     // the last call's condition lists
+  const uint32_t* bc_dof = nullptr;    // in bc_upload: bc_n dofs and their last values
+  const double* bc_vlast = nullptr;
   DevBuf bc_vfirst;     // double dofs (valid at BC dofs)
   DevBuf bc_mask;       // uint8 n_nodes: bit e set when dof (node, e) carries a condition
   DevBuf bc_newmask;    // uint8 n_nodes: conditions added by the current call
@@ -265,6 +270,7 @@ size_t batch_table_bytes(uint32_t max_cases);                    // assembly.hip
 void batch_assemble(Batch& B, uint32_t n, Lss* const* L, Fields* const* F, const cf3hip_ns_params* prm);
 
 // lss.hip
+void lss_forget_conditions(Lss& L);   // host side of lss_clear_conditions
 void lss_fill(Context& c, double* p, size_t n, double v);
 void lss_fill32(Context& c, float* p, size_t n, float v);
 void lss_round_fp32(Lss& L);   // values32 = fl32(values)

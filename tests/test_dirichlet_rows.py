@@ -1,0 +1,60 @@
+"""Symmetric Dirichlet conditions on ragged rows (shorter and longer than the 16 blocks a lane group takes at
+once) against the oracle: several calls between resets, dofs repeated within and across calls, every dof of a
+node or one of them, and a reset in between.
+
+Bar: values exactly (entries are kept, zeroed or set to 1); rhs within (blocks of a row x neq + 2) eps of the
+sum of the absolute terms, whose order is the kernel's own."""
+import numpy as np
+import pytest
+
+from coolfluid3_amd import cabi
+
+pytestmark = pytest.mark.gpu
+
+
+def symmetric_graph(N, seed):
+    rng = np.random.default_rng(seed)
+    a = np.eye(N, dtype=bool)
+    a[0, :] = a[:, 0] = True                       # a hub: one row as long as the system
+    for i, j in rng.integers(0, N, (3 * N, 2)):
+        a[i, j] = a[j, i] = True
+    rows = [np.flatnonzero(r) for r in a]
+    start = np.concatenate([[0], np.cumsum([len(r) for r in rows])])
+    return start.astype(np.uint32), np.concatenate(rows).astype(np.uint32)
+
+
+@pytest.mark.parametrize("neq", [1, 2, 3, 4])
+@pytest.mark.parametrize("N", [1, 17, 200])
+def test_conditions_against_oracle(oracle, neq, N):
+    print("neq", neq, "N", N, flush=True)
+    start, cols = symmetric_graph(N, N + neq)
+    rng = np.random.default_rng(N)
+    ctx = cabi.Context(0)
+    s = cabi.System(ctx, neq=neq, graph=(start, cols, N))
+    n = int(start[-1])
+    for _ in range(2):                              # the second round after a reset
+        s.reset(0.0)
+        for i in range(N):                          # distinct values, one block row at a time
+            idx = cols[start[i]:start[i + 1]]
+            for c in idx:
+                s.set_value(int(c) * neq + int(rng.integers(neq)), i * neq + int(rng.integers(neq)), rng.uniform(-2, 2))
+        vals = s.values()
+        rhs, sol = rng.uniform(-1, 1, N * neq), rng.uniform(-1, 1, N * neq)
+        s.set_vector(cabi.RHS, rhs)
+        s.set_vector(cabi.SOLUTION, sol)
+        scale = np.abs(rhs) + 3 * np.abs(vals).max() * np.diff(start.astype(np.int64)).max() * neq
+        for call in range(3):
+            k = max(1, N // 4)
+            nodes = rng.integers(0, N, k).astype(np.uint32)
+            nodes = np.concatenate([nodes, nodes[:2], np.zeros(1 if call == 1 else 0, np.uint32)]).astype(np.uint32)
+            eqs = rng.integers(0, neq, len(nodes)).astype(np.uint32)
+            v = rng.uniform(-1, 1, len(nodes))
+            s.dirichlet(nodes, eqs, v)
+            oracle.dirichlet(neq, start, cols, vals, rhs, sol, nodes, eqs, v)
+            assert np.array_equal(s.values(), vals)
+            assert np.array_equal(s.vector(cabi.SOLUTION), sol)
+            bar = (np.diff(start.astype(np.int64)).max() * neq + 2) * 2.0 ** -52 * scale
+            assert (np.abs(s.vector(cabi.RHS) - rhs) <= bar).all()
+    assert n == s.n_blocks
+    s.close()
+    ctx.close()
