@@ -35,7 +35,7 @@ struct AsmArgs {
   double c1, c2, a_ps, a_su, a_bu;
   double u_ref;        // CF2 reference velocity
   int* status;         // 1: non-positive Jacobian determinant, 2: CF2 element Reynolds number not positive
-  double* q1rec;       // Q1 cells: per element and Gauss point J^-1, det J, u_adv, nu (Q1Rec doubles)
+  double* q1rec;       // Q1 cells: J^-1, det J, u_adv, nu of the Gauss points, (element, entry pair, point, 2)
   double4* q1tau;      // Q1 cells: per element (tau_ps, tau_su, tau_bulk, 0)
 };
 
