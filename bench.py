@@ -549,7 +549,7 @@ def main():
         "fp32_assembly_Melem_s": E / a32_kern / 1e3,
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                     "kernel": "k_assemble<SpecP1<3,double>>", "algorithmic_bytes": alg,
+                     "kernel": "k_assemble_lists<3,double,true>", "algorithmic_bytes": alg,
                      "kernel_ms": kern_ms},
         "extra": extra,
     }

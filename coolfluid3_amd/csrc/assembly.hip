@@ -726,10 +726,10 @@ __global__ __launch_bounds__(kThreads, sizeof(R) == sizeof(float) ? 5 : 1) void 
 // combine and the rhs product for every one.
 // Measured (kernel, us, staged reduction -> block lists): FP64 tetrahedra 61^3 cells 389 -> 264, 128^3
 // 3147 -> 2179; FP32 208 -> 143, 1811 -> 1139; triangles 700^2 140 -> 120 (FP64), 81 -> 68 (FP32).
-// At 61^3: 1206 -> 990 VALU instructions per wave and 5/6 of the waves, 25 % fewer LDS instructions; VALU and LDS are each
-// busy about 60 % of the time with 5 to 6 workgroups per CU, and neither HBM (1.9 TB/s) nor the load chain at
-// the start bounds it: a persistent form that loads the next plan and its nodes during the block sums was no
-// faster (its 159 VGPRs cost the waves that hid the same latency).
+// At 61^3: 1206 -> 990 VALU instructions per wave and 5/6 of the waves, 25 % fewer LDS instructions; VALU and
+// LDS are each busy about 60 % of the time with 5 to 6 workgroups per CU, and neither HBM (1.9 TB/s) nor the
+// load chain at the start bounds it: a persistent form that loads the next plan and its nodes during the block
+// sums was no faster (its 159 VGPRs cost the waves that hid the same latency).
 // dynamic LDS: [nodal states] [other nodal data; then the element records; then the block rows and rhs
 // parts], the states kept to the end with RHS.  The nodal data are arrays of 16-byte pairs, (u, v), (w, p),
 // (x, y), (z, nu), (u_adv x, y), and u_adv z: whole 32-byte records would put every first half on the same

@@ -168,8 +168,7 @@ __device__ inline bool leader() { return blockIdx.x == 0 && threadIdx.x == 0; }
 // Elements a thread of the vector kernels has in flight.  Its first ones are loaded before the scalars of the
 // iteration are known: on small systems a launch is one chain of load, reduction and update, so every load
 // that can start at once does.  Measured per launch (p / s / x update, us): 16 k rows of one equation
-// 4.5 / 3.9 / 5.1 -> 4.0 / 3.7 / 5.2; 64^3 tetrahedra
-// 14.0 / 13.1 / 21.3 -> 11.6 / 11.0 / 20.4.
+// 4.5 / 3.9 / 5.1 -> 4.0 / 3.7 / 5.2; 64^3 tetrahedra 14.0 / 13.1 / 21.3 -> 11.6 / 11.0 / 20.4.
 constexpr int kVecU = 4;
 
 template<typename R>
@@ -782,9 +781,9 @@ void read_scalars(Context& c, Scalars& s)
 
 // Device state of one BiCGStab recurrence (Jacobi right preconditioning, dinv = D^-1) and the launches
 // that advance it; the scalars stay on the device and the host reads them once per batch.  With FP64
-// vectors and neq = 1 to 4 an iteration is five launches (dot products fused into the products, each
-// reduction completed by the kernel that consumes it); otherwise eleven (separate dot products and
-// one-workgroup finalisations).  Both sum in a fixed order: the results are deterministic.  rel selects
+// vectors and neq = 1 to 4 an iteration is five launches, on small systems three (dot products fused into
+// the products, each reduction completed by the kernel that consumes it); otherwise eleven (separate dot
+// products and one-workgroup finalisations).  Both sum in a fixed order: the results are deterministic.  rel selects
 // the residual-replacement stop test of the reliable phase.
 template<typename R, typename VR>
 struct Recurrence {
