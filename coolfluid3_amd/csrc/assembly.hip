@@ -752,8 +752,35 @@ struct PlanLayout {
   }
 };
 
-template<int D, typename R, bool RHS>
-__device__ __forceinline__ void assemble_lists_wg(const AsmArgs& g, uint32_t wg, unsigned char* smem)
+// the fields of a system, and the node records that the packing kernels write from them
+struct PackArgs {
+  const double* u[3];
+  const double* ua[3];
+  const double* p;
+  const double* nu;
+  double4* st;
+  double4* ad;
+};
+
+template<int D>
+__device__ __forceinline__ void read_node(const PackArgs& f, uint64_t i, double4& st, double4& ad)
+{
+  if constexpr(D == 3) {
+    st = make_double4(f.u[0][i], f.u[1][i], f.u[2][i], f.p[i]);
+    ad = make_double4(f.ua[0][i], f.ua[1][i], f.ua[2][i], f.nu[i]);
+  } else {
+    st = make_double4(f.u[0][i], f.u[1][i], f.p[i], 0.);
+    ad = make_double4(f.ua[0][i], f.ua[1][i], 0., f.nu[i]);
+  }
+}
+
+// DIRECT: the nodes' states come from the field arrays, otherwise from the packed records (the batched launch,
+// whose pass over all systems packs them).  A plan reads a node once, so the packing pass, a launch of its own,
+// costs more than the eight loads per node it saves: linearise + assemble + product, records -> fields, us: 32^2 x 2
+// triangles 26.0 -> 23.1; FP32 tetrahedra 23^3 cells 32.7 -> 29.4, 100^3 814 -> 790; FP64 61^3 353 -> 345, 128^3
+// 3001 -> 2972.
+template<int D, typename R, bool RHS, bool DIRECT>
+__device__ __forceinline__ void assemble_lists_wg(const AsmArgs& g, const PackArgs& f, uint32_t wg, unsigned char* smem)
 {
   typedef PlanLayout<D, R> Y;
   constexpr int K = Y::K, NEQ = Y::NEQ, NN = Y::NN, LDW = Y::LDW;
@@ -782,7 +809,14 @@ __device__ __forceinline__ void assemble_lists_wg(const AsmArgs& g, uint32_t wg,
   R* s_rhs = s_row + LDW * g.plan_lists;
   for(uint32_t j = t; j < ns; j += kThreads) {
     const uint32_t nd = nodes[j];
-    const double4 xp = g.xp[nd], st = g.st[nd], ad = g.ad[nd];
+    const double4 xp = g.xp[nd];
+    double4 st, ad;
+    if constexpr(DIRECT) {
+      read_node<D>(f, nd, st, ad);
+    } else {
+      st = g.st[nd];
+      ad = g.ad[nd];
+    }
     s_xy[j] = make_double2(xp.x, xp.y);
     s_zn[j] = make_double2(xp.z, ad.w);
     s_uv[j] = make_double2(st.x, st.y);
@@ -987,25 +1021,16 @@ __device__ __forceinline__ void assemble_lists_wg(const AsmArgs& g, uint32_t wg,
 }
 
 template<int D, typename R, bool RHS>
-__global__ __launch_bounds__(kThreads, sizeof(R) == sizeof(float) ? 4 : 3) void k_assemble_lists(AsmArgs g)
+__global__ __launch_bounds__(kThreads, sizeof(R) == sizeof(float) ? 4 : 3) void k_assemble_lists(AsmArgs g, PackArgs f)
 {
   extern __shared__ double4 s_dyn[];
-  assemble_lists_wg<D, R, RHS>(g, xcd_order(blockIdx.x, gridDim.x), reinterpret_cast<unsigned char*>(s_dyn));
+  assemble_lists_wg<D, R, RHS, true>(g, f, xcd_order(blockIdx.x, gridDim.x), reinterpret_cast<unsigned char*>(s_dyn));
 }
 
 // ---------------------------------------------------------------------------------------------
 // Batched FP32 assembly of many tetrahedral systems (serving): one persistent launch whose
 // workgroups walk the concatenated workgroup lists of the systems in a device table.
 // ---------------------------------------------------------------------------------------------
-struct PackArgs {
-  const double* u[3];
-  const double* ua[3];
-  const double* p;
-  const double* nu;
-  double4* st;
-  double4* ad;
-};
-
 struct BatchEntry {
   AsmArgs g;
   PackArgs pk;
@@ -1046,7 +1071,7 @@ __global__ __launch_bounds__(kThreads) void k_batch_assemble(const BatchHeader* 
   for(uint32_t task = blockIdx.x; task < total; task += gridDim.x) {
     __syncthreads();   // the previous task's LDS reads are done
     const uint32_t c = batch_find(e, n, task, true);
-    assemble_lists_wg<3, float, false>(e[c].g, task - e[c].wg_begin, reinterpret_cast<unsigned char*>(s_dyn));
+    assemble_lists_wg<3, float, false, false>(e[c].g, e[c].pk, task - e[c].wg_begin, reinterpret_cast<unsigned char*>(s_dyn));
   }
 }
 
@@ -1130,21 +1155,16 @@ __global__ void k_pack_fields(uint32_t n, PackArgs a)
 {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if(i >= n) return;
-  if constexpr(D == 3) {
-    a.st[i] = make_double4(a.u[0][i], a.u[1][i], a.u[2][i], a.p[i]);
-    a.ad[i] = make_double4(a.ua[0][i], a.ua[1][i], a.ua[2][i], a.nu[i]);
-  } else {
-    a.st[i] = make_double4(a.u[0][i], a.u[1][i], a.p[i], 0.);
-    a.ad[i] = make_double4(a.ua[0][i], a.ua[1][i], 0., a.nu[i]);
-  }
+  double4 st, ad;
+  read_node<D>(a, i, st, ad);
+  a.st[i] = st;
+  a.ad[i] = ad;
 }
 
-void pack_fields(Fields& F)
+PackArgs field_args(Fields& F)
 {
-  const Mesh& M = *F.mesh;
-  Context& c = *M.ctx;
   PackArgs a = {};
-  for(int d = 0; d < M.dim; ++d) {
+  for(int d = 0; d < F.mesh->dim; ++d) {
     a.u[d] = F.u[d].as<double>();
     a.ua[d] = F.uadv[d].as<double>();
   }
@@ -1152,6 +1172,14 @@ void pack_fields(Fields& F)
   a.nu = F.nu.as<double>();
   a.st = F.st.as<double4>();
   a.ad = F.ad.as<double4>();
+  return a;
+}
+
+void pack_fields(Fields& F)
+{
+  const Mesh& M = *F.mesh;
+  Context& c = *M.ctx;
+  const PackArgs a = field_args(F);
   if(M.dim == 3) hipLaunchKernelGGL(k_pack_fields<3>, dim3(grid_for(M.n_nodes, 256)), dim3(256), 0, c.stream, M.n_nodes, a);
   else hipLaunchKernelGGL(k_pack_fields<2>, dim3(grid_for(M.n_nodes, 256)), dim3(256), 0, c.stream, M.n_nodes, a);
   HIP_OK(hipGetLastError());
@@ -1170,16 +1198,17 @@ void launch(const AsmArgs& g, const Lss& L)
 // specialised simplices: by block lists; a system without plans (a workgroup that touches more than
 // kPlanNodes nodes, or a node with too many elements) takes the staged reduction
 template<int D, typename R, bool RHS>
-void launch_spec(const AsmArgs& g, const Lss& L)
+void launch_spec(const AsmArgs& g, const Lss& L, Fields& F)
 {
   if(!g.plan) {
+    pack_fields(F);
     launch<SpecP1<D, R>, R, R, RHS>(g, L);
     return;
   }
   Context& c = *L.ctx;
   const size_t lds = PlanLayout<D, R>::lds_bytes(RHS, L.plan_nodes, L.plan_elems, L.plan_lists);
   timer_begin(c, CF3HIP_KERNEL_ASSEMBLY);
-  hipLaunchKernelGGL((k_assemble_lists<D, R, RHS>), dim3(L.n_plan), dim3(kThreads), lds, c.stream, g);
+  hipLaunchKernelGGL((k_assemble_lists<D, R, RHS>), dim3(L.n_plan), dim3(kThreads), lds, c.stream, g, field_args(F));
   HIP_OK(hipGetLastError());
   timer_end(c, CF3HIP_KERNEL_ASSEMBLY);
 }
@@ -1261,11 +1290,12 @@ void mesh_pack_coords(Mesh& M)
 
 void assemble(Lss& L, Fields& F, const cf3hip_ns_params& prm)
 {
-  AsmArgs g = make_args(L, F, prm);
+  // the specialised kernels read the fields themselves or pack them in launch_spec
+  const bool spec = L.mesh && prm.use_specializations && !is_cell(L.mesh->etype);
+  AsmArgs g = make_args(L, F, prm, !spec);
   const Mesh& M = *L.mesh;
   if(prm.precision == CF3HIP_FP32 && !L.has_fp32)
     CF3_THROW(CF3HIP_ERR_NOT_CREATED, "FP32 assembly needs cf3hip_lss_enable_fp32");
-  const bool spec = prm.use_specializations && !is_cell(M.etype);
   Context& c = *L.ctx;
   const bool fp32 = prm.precision == CF3HIP_FP32;
   // ZeroLSS: every value and rhs entry is overwritten by the kernel; the conditions of the previous
@@ -1281,11 +1311,11 @@ void assemble(Lss& L, Fields& F, const cf3hip_ns_params& prm)
   if(is_cell(M.etype)) {
     launch_hex(g, L, fp32 ? 1 : 0);
   } else if(spec && M.etype == CF3HIP_TETRA3D) {
-    if(fp32) launch_spec<3, float, false>(g, L);
-    else launch_spec<3, double, true>(g, L);
+    if(fp32) launch_spec<3, float, false>(g, L, F);
+    else launch_spec<3, double, true>(g, L, F);
   } else if(spec && M.etype == CF3HIP_TRIAG2D) {
-    if(fp32) launch_spec<2, float, false>(g, L);
-    else launch_spec<2, double, true>(g, L);
+    if(fp32) launch_spec<2, float, false>(g, L, F);
+    else launch_spec<2, double, true>(g, L, F);
   } else if(M.etype == CF3HIP_TETRA3D) {
     if(fp32) launch<GenericP1<3>, double, float, false>(g, L);
     else launch<GenericP1<3>, double, double, true>(g, L);
