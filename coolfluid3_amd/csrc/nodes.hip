@@ -11,7 +11,7 @@ namespace {
 #pragma clang fp contract(off)
 
 // the components of a field history, one launch for all of them (blockIdx.y): on small meshes a launch costs
-// its latency (linearise + assemble on 32^2 x 2 triangles 28.0 -> 26.5 us, on 23^3 x 5 FP32 tetrahedra
+// its latency (linearise + assemble on 32^2 x 2 triangles 28.0 -> 26.5 us, on 23^3 x 6 FP32 tetrahedra
 // 36.0 -> 33.4 us)
 struct History {
   double *u[3], *u1[3], *u2[3], *u3[3], *ua[3];
