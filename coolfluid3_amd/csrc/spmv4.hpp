@@ -51,6 +51,9 @@ __device__ __forceinline__ double row_f64(const uint32_t* __restrict__ row_ptr, 
 
 // FP32 values, FP64 vectors and accumulation: lane l streams one block row (4 floats, 16 B) of
 // blocks 4k + (l >> 2), component l & 3; lanes l < 4 hold y[row * 4 + l] after the call.
+// One block per trip: with 12 doubles a block in flight, four cost more waves than they hide latency.  Per iteration of
+// the precision form (two products and the vector kernels), four -> two -> one, us: 100^3 tetrahedra 746 -> 725 -> 694;
+// hexahedra 100^3 1308 with two, 1220 with one; 37^3 and 60^3 tetrahedra equal within 1 %.
 __device__ __forceinline__ double row_mixed(const uint32_t* __restrict__ row_ptr, const uint32_t* __restrict__ cols,
                                             const float* __restrict__ vals, const double* __restrict__ x,
                                             uint32_t row, int l, int& a, bool& out)
@@ -59,23 +62,11 @@ __device__ __forceinline__ double row_mixed(const uint32_t* __restrict__ row_ptr
   const int sub = l >> 2;
   a = l & 3;
   double acc = 0.;
-  for(uint32_t q = q0 + sub; q < q1; q += 4 * kTrip) {
-    float4 v[kTrip];
-    double2 x01[kTrip], x23[kTrip];
-#pragma unroll
-    for(int k = 0; k < kTrip; ++k) {
-      const uint32_t qq = min(q + 4u * k, q1 - 1);
-      const double2* xb = reinterpret_cast<const double2*>(x + (uint64_t)cols[qq] * 4);
-      v[k] = *reinterpret_cast<const float4*>(vals + (uint64_t)qq * 16 + 4 * a);
-      x01[k] = xb[0];
-      x23[k] = xb[1];
-    }
-#pragma unroll
-    for(int k = 0; k < kTrip; ++k) {
-      const double s = (double)v[k].x * x01[k].x + (double)v[k].y * x01[k].y + (double)v[k].z * x23[k].x +
-                       (double)v[k].w * x23[k].y;
-      acc = q + 4u * k < q1 ? acc + s : acc;
-    }
+  for(uint32_t q = q0 + sub; q < q1; q += 4) {
+    const double2* xb = reinterpret_cast<const double2*>(x + (uint64_t)cols[q] * 4);
+    const float4 v = *reinterpret_cast<const float4*>(vals + (uint64_t)q * 16 + 4 * a);
+    const double2 x01 = xb[0], x23 = xb[1];
+    acc += (double)v.x * x01.x + (double)v.y * x01.y + (double)v.z * x23.x + (double)v.w * x23.y;
   }
   acc += lanes::move<lanes::kNext4>(acc);
   acc += lanes::move<lanes::kNext8>(acc);
