@@ -114,49 +114,55 @@ __global__ void k_spmv_mixed_generic(uint32_t N, int neq, const uint32_t* __rest
   y[r] = acc;
 }
 
-// neq = 2 or 3 (values VR, vectors T): a workgroup owns kStreamRows node rows and streams their values as one
+// neq = 2 or 3 (values VR, vectors T): a workgroup owns stream_rows node rows and streams their values as one
 // contiguous array, consecutive lanes on consecutive values (a block of 4 or 9 values is no multiple of a
-// 16-byte load, and one thread per scalar row reads it with a stride of a whole row).  The products go to
-// LDS; one thread per scalar row then sums its own, blocks in ascending order.  A range of more than
-// kStreamBlocks blocks is taken in pieces.  Bound by the value stream; 512 x 512 quadrilaterals, neq = 3,
-// 180 MB: 93 us with one thread per scalar row, 44 us (4.4 TB/s).
-constexpr int kStreamRows = 24;     // x 9 blocks of a quadrilateral mesh = 216
-constexpr int kStreamBlocks = 256;
+// 16-byte load, and one thread per scalar row reads it with a stride of a whole row).  Values and gathered x go
+// to LDS as they are; one thread per scalar row then sums its own by fused multiply-adds, blocks and columns in
+// ascending order: bit for bit the sums of k_spmv_generic.  A range of more than stream_blocks blocks is taken
+// in pieces.  Bound by the value stream where enough workgroups fit into LDS: 512 x 512 quadrilaterals, neq = 3,
+// 180 MB, one thread per scalar row 93 us; 24 rows and 256 blocks (24 KB) 51 us, 216 blocks 46.7, 14 rows and 128
+// blocks 42 us (4.6 TB/s); 500^2 x 2 triangles 37.4 / 34.1 / 35.6.  FP32 (34.7 against 37.7 us) keeps the large ones.
+template<typename T> constexpr int stream_rows() { return sizeof(T) == 8 ? 14 : 24; }   // x 9 blocks of a quadrilateral mesh
+template<typename T> constexpr int stream_blocks() { return sizeof(T) == 8 ? 128 : 256; }
 template<typename T, typename VR, int NEQ>
 __global__ __launch_bounds__(256) void k_spmv_stream(uint32_t N, const uint32_t* __restrict__ row_ptr,
                                                      const uint32_t* __restrict__ cols, const VR* __restrict__ vals,
                                                      T alpha, const T* __restrict__ x, T beta, T* __restrict__ y,
                                                      const double* __restrict__ stop)
 {
-  constexpr int NN = NEQ * NEQ;
-  __shared__ T s_prod[kStreamBlocks * NN];
+  constexpr int NN = NEQ * NEQ, ROWS = stream_rows<T>(), BLOCKS = stream_blocks<T>();
+  constexpr int TRIPS = (BLOCKS * NEQ + 255) / 256, VTRIPS = (BLOCKS * NN + 255) / 256;
+  __shared__ VR s_val[BLOCKS * NN];
+  __shared__ T s_x[BLOCKS * NEQ];
   if(stop && stop[0] != 0.) return;
   const uint32_t t = threadIdx.x;
-  const uint32_t row0 = blockIdx.x * kStreamRows;
-  const uint32_t nr = min((uint32_t)kStreamRows, N - row0);
+  const uint32_t row0 = blockIdx.x * ROWS;
+  const uint32_t nr = min((uint32_t)ROWS, N - row0);
   const uint32_t b0 = row_ptr[row0], b1 = row_ptr[row0 + nr];
   const bool owner = t < nr * NEQ;
   const uint32_t i = t / NEQ, a = t % NEQ;
   uint32_t q0 = 0, q1 = 0;
   if(owner) { q0 = row_ptr[row0 + i]; q1 = row_ptr[row0 + i + 1]; }
   T acc = T(0);
-  for(uint32_t c0 = b0; c0 < b1; c0 += kStreamBlocks) {
-    const uint32_t nb = min((uint32_t)kStreamBlocks, b1 - c0);
+  for(uint32_t c0 = b0; c0 < b1; c0 += BLOCKS) {
+    const uint32_t nb = min((uint32_t)BLOCKS, b1 - c0);
     if(c0 != b0) __syncthreads();   // the sums of the previous piece are taken
 #pragma unroll
-    for(int k = 0; k < NN; ++k) {
+    for(int k = 0; k < TRIPS; ++k) {
       const uint32_t e = t + 256u * k;
-      if(e < nb * NN) {
-        const uint32_t q = e / NN, c = e % NEQ;   // NN is a multiple of NEQ
-        s_prod[e] = (T)vals[(uint64_t)c0 * NN + e] * x[(uint64_t)cols[c0 + q] * NEQ + c];
-      }
+      if(e < nb * NEQ) s_x[e] = x[(uint64_t)cols[c0 + e / NEQ] * NEQ + e % NEQ];
+    }
+#pragma unroll
+    for(int k = 0; k < VTRIPS; ++k) {
+      const uint32_t e = t + 256u * k;
+      if(e < nb * NN) s_val[e] = vals[(uint64_t)c0 * NN + e];
     }
     __syncthreads();
     if(owner) {
       const uint32_t lo = max(q0, c0), hi = min(q1, c0 + nb);
       for(uint32_t q = lo; q < hi; ++q)
 #pragma unroll
-        for(int b = 0; b < NEQ; ++b) acc += s_prod[(q - c0) * NN + a * NEQ + b];
+        for(int b = 0; b < NEQ; ++b) acc += (T)s_val[(q - c0) * NN + a * NEQ + b] * s_x[(q - c0) * NEQ + b];
     }
   }
   if(owner) {
@@ -331,7 +337,7 @@ namespace {
 template<typename T, typename VR>
 void spmv_stream(Lss& L, const VR* vals, T alpha, const T* x, T beta, T* y, const double* stop)
 {
-  const dim3 g(grid_for(L.n_nodes, kStreamRows));
+  const dim3 g(grid_for(L.n_nodes, stream_rows<T>()));
   const uint32_t* rp = L.row_ptr.as<uint32_t>();
   const uint32_t* cl = L.cols.as<uint32_t>();
   if(L.neq == 2)

@@ -61,3 +61,38 @@ def test_product_on_ragged_rows(neq, N):
         assert (np.abs(got - (alpha * d32 @ x32.astype(np.float64) + beta * y32)) <= bar).all()
     s.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("neq", [1, 2, 3])
+def test_products_are_fused(neq):
+    """Row sums are fused multiply-adds in ascending order: with a a = 1 + 2 e + e^2, whose last term the rounded
+    product drops, -(1 + 2 e) 1 + a a leaves exactly e^2."""
+    print("neq", neq, flush=True)
+    N = 30
+    other = np.maximum(np.arange(N), 1)                              # row 0: columns 0 and 1; row i: 0 and i
+    cols = np.stack([np.zeros(N), other], axis=1).ravel().astype(np.uint32)
+    ctx = cabi.Context(0)
+    s = cabi.System(ctx, neq=neq, graph=(np.arange(N + 1, dtype=np.uint32) * 2, cols, N))
+    s.enable_fp32()
+    for e, dtype in ((2.0 ** -30, np.float64), (2.0 ** -13, np.float32)):
+        s.reset(0.0)
+        x = np.ones(N * neq)
+        for i in range(N):
+            for k in range(neq):
+                s.set_value(k, i * neq + k, -(1 + 2 * e))
+                s.set_value(int(other[i]) * neq + k, i * neq + k, 1 + e)
+                x[other[i] * neq + k] = 1 + e
+        if dtype == np.float64:
+            s.set_vector(cabi.SOLUTION, x)
+            s.apply_device(1.0, s.vector_ptr(cabi.SOLUTION), 0.0, s.vector_ptr(cabi.RHS))
+            y = s.vector(cabi.RHS)
+        else:
+            s.round_fp32()
+            pad = np.zeros(2 * N * neq, np.float32)
+            pad[:N * neq] = x
+            s.set_vector(cabi.SOLUTION, pad.view(np.float64))
+            s.apply_fp32_device(1.0, s.vector_ptr(cabi.SOLUTION), 0.0, s.vector_ptr(cabi.RHS))
+            y = s.vector(cabi.RHS).view(np.float32)[:N * neq]
+        assert (y == e * e).all()
+    s.close()
+    ctx.close()
