@@ -529,10 +529,12 @@ __global__ __launch_bounds__(kRT) void k_fb_product(uint32_t N, const uint32_t* 
         for(int j = 0; j < CW; ++j) x[j] = gd[k][j] * update(gr[k][j], STAGE == 1 ? gp[k][j] : 0., gv[k][j]);
 #pragma unroll
         for(int i = 0; i < RW; ++i) {
-          double sum = m[k][i][0] * x[0];
+          // a lane's blocks of a row are one chain of fused multiply-adds; WIDE: the two columns first, as row_f64
+          double sum = WIDE ? m[k][i][0] * x[0] : ys[i] + m[k][i][0] * x[0];
 #pragma unroll
           for(int j = 1; j < CW; ++j) sum += m[k][i][j] * x[j];
-          ys[i] = q + BL * k < q1 ? ys[i] + sum : ys[i];
+          if constexpr(WIDE) sum += ys[i];
+          ys[i] = q + BL * k < q1 ? sum : ys[i];
         }
       }
       q += BL * T;

@@ -56,3 +56,32 @@ def test_solves_across_sizes(neq, N):
         assert st.converged and residual(s.vector(cabi.SOLUTION)) <= 10 * tol
     s.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("neq", [1, 2, 3])
+def test_products_are_fused(neq):
+    """The row sums of the three-launch iteration are fused multiply-adds: row 0 is the identity and two couplings of
+    one lane (8 or 16 blocks apart) whose products with the first direction, -(1 + 2 e) and (1 + e)^2, leave e^2
+    (rounded products leave nothing).  All other rows are identities, so alpha = omega = 1 and the first iteration
+    ends with x_0 = -e^2."""
+    print("neq", neq, flush=True)
+    N, far, e = 40, 1 + (8 if neq == 1 else 16), 2.0 ** -30
+    rows = [np.arange(N)] + [np.array([0, i]) for i in range(1, N)]
+    start = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.uint32)
+    ctx = cabi.Context(0)
+    s = cabi.System(ctx, neq=neq, graph=(start, np.concatenate(rows).astype(np.uint32), N))
+    s.reset(0.0)
+    for i in range(N * neq):
+        s.set_value(i, i, 1.0)
+    s.set_value(neq, 0, -(1 + 2 * e))
+    s.set_value(far * neq, 0, 1 + e)
+    b = np.zeros(N * neq)
+    b[neq], b[far * neq] = 1.0, 1 + e
+    s.set_vector(cabi.RHS, b)
+    s.reset_vector(cabi.SOLUTION)
+    s.solve(cabi.solver_params(tol=1e-60, max_iter=1), raise_on_failure=False)
+    x = s.vector(cabi.SOLUTION)
+    b[0] = -e * e
+    assert np.array_equal(x, b)
+    s.close()
+    ctx.close()
