@@ -49,7 +49,7 @@ struct SpecP1 {
   R ua[D];          // mean advection velocity u_avg
   R na[D];          // normal of the row node a
   R Q[D];           // velocity-row coefficient: skew-symmetric advection + stress diffusion + bulk
-  R tsdV, nudV, visc, m0dt;   // element: tau / (D^2 V), nu / (D^2 V), nu / (3 D^2 V) + tau_bulk / (D^2 V), V / (12|20 dt)
+  R tsdV, nudV, visc, m0;   // element: tau / (D^2 V), nu / (D^2 V), nu / (3 D^2 V) + tau_bulk / (D^2 V), V / (12|20)
   R tsu;
   R cc, cpres, pn, pp, tdo, tdd, tpc;
   int a;
@@ -105,9 +105,9 @@ struct SpecP1 {
         gsq += (i == l ? T(1) : T(2)) * gil * gil;
         if(i == l) tr += gil;
       }
-    const T q = f4dt2 + adv + T(16) * (nu * nu * gsq);
-    t_su = inv_sqrt(q);
-    t_bu = (q * t_su) * reciprocal(tr);
+    const T sq = sqrt(f4dt2 + adv + T(16) * (nu * nu * gsq));
+    t_su = T(1) / sq;
+    t_bu = sq / tr;
   }
 
   __device__ __forceinline__ void prepare(const AsmArgs& g, uint32_t e, int a_)
@@ -177,7 +177,7 @@ struct SpecP1 {
     if(fp64_geom) {
       double n64[K][D], V64, ts, tb;
       geometry<double>(X, n64, V64);
-      const double iv = reciprocal(V64);
+      const double iv = 1. / V64;
       tau_metric<double>(n64, iv * (1.0 / D), uc, nu_mean, g.f4dt2, ts, tb);
       for(int m = 0; m < K; ++m)
         for(int d = 0; d < D; ++d) n[m][d] = (R)n64[m][d];
@@ -188,12 +188,12 @@ struct SpecP1 {
         // det J of the Jacobian, as the reference's ComputeTau does (SUPG.hpp:178, ElementData.hpp:302-314)
         const double Vr = tet_volume_ref(X);
         V = Vr;
-        invV = reciprocal(Vr);
+        invV = 1. / Vr;
       }
     } else {
       R ucr[D];
       for(int d = 0; d < D; ++d) ucr[d] = (R)uc[d];
-      invV = reciprocal(V);
+      invV = R(1) / V;
       tau_metric<R>(n, invV * R(1.0 / D), ucr, nu, (R)g.f4dt2, tsu, tbu);
       if(!(V > R(0))) g.status[0] = 1;
     }
@@ -201,7 +201,7 @@ struct SpecP1 {
     tsdV = tsu * rdV;
     nudV = nu * rdV;
     visc = nudV * R(1.0 / 3.0) + tbu * rdV;
-    m0dt = (R)g.invdt * (V * R(D == 2 ? 1.0 / 12.0 : 1.0 / 20.0));
+    m0 = V * R(D == 2 ? 1.0 / 12.0 : 1.0 / 20.0);
   }
 
   // coefficients of the row of local node a_
@@ -236,8 +236,8 @@ struct SpecP1 {
     pn = R(0.5) * tsdV * ni_ut + c0;   // tau_ps = tau_su
     pp = tsdV * inv_rho;
     const R invdt = (R)g.invdt;
-    tdo = m0dt + invdt * time_ii;
-    tdd = tdo + m0dt;
+    tdo = invdt * (m0 + time_ii);
+    tdd = invdt * (R(2) * m0 + time_ii);
     tpc = invdt * tsu * c0;
   }
 
@@ -863,7 +863,7 @@ __device__ __forceinline__ void assemble_lists_wg(const AsmArgs& g, const PackAr
     rec[Y::ELEM + 2] = op.visc;
     rec[Y::ELEM + 3] = op.ua[0];
     rec[Y::ELEM + 4] = op.ua[1];
-    rec[Y::ELEM + 5] = op.m0dt;
+    rec[Y::ELEM + 5] = (R)g.invdt * op.m0;
   }
   if(t < (uint32_t)Y::WORDS) s_rec[ne * Y::STRIDE + t] = R(0);   // the record of the unused list entries
   // block of this thread's list; row of the LDS rows: the first list of a block at its block, the others

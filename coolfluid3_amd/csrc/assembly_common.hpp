@@ -81,25 +81,6 @@ __device__ __forceinline__ double tet_volume_ref(const double X[4][3])
           x0*y1*z3 - x2*y1*z3 - x0*y2*z3 + x1*y2*z3) / 6.;
 }
 
-// 1 / x and 1 / sqrt(x) for positive normal x by Newton steps from the hardware estimates: within an ulp or
-// two, in 5 and 9 FP64 instructions against 11 and about 25 of the correctly rounded division and root (the
-// element quantities take four of them per element).  Zero, negative, infinite and NaN arguments give what
-// the callers' Jacobian test reports or a NaN.
-__device__ __forceinline__ double reciprocal(double x)
-{
-  double r = __builtin_amdgcn_rcp(x);
-  r = fma(fma(-x, r, 1.), r, r);
-  return fma(fma(-x, r, 1.), r, r);
-}
-__device__ __forceinline__ float reciprocal(float x) { return 1.f / x; }
-__device__ __forceinline__ double inv_sqrt(double x)
-{
-  double r = __builtin_amdgcn_rsq(x);
-  r = fma(0.5 * r, fma(-x * r, r, 1.), r);
-  return fma(0.5 * r, fma(-x * r, r, 1.), r);
-}
-__device__ __forceinline__ float inv_sqrt(float x) { return 1.f / sqrtf(x); }
-
 // one LDS row of a staged element block: 16-byte aligned, odd number of 16-byte chunks (bank spread)
 template<typename VR, int NN>
 constexpr int lds_row()

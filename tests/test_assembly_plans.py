@@ -89,3 +89,29 @@ def test_periodic_blocks_of_several_nodes(ctx, oracle, etype, n):
     assert np.abs(g.system.values() - vref).max() <= 1e-12 * np.abs(vref).max()
     assert np.abs(g.system.vector(cabi.RHS) - rref).max() <= 1e-12 * np.abs(rref).max()
     g.close()
+
+
+@pytest.mark.parametrize("etype", [cabi.TRIAG2D, cabi.TETRA3D])
+def test_infinite_tau_argument(ctx, oracle, etype):
+    """Velocities whose squares overflow: tau = 1 / sqrt(inf) = 0, so a continuity row is the divergence sum over
+    elements of V / (dim + 1) grad N_b alone, and finite (the momentum rows hold tau_bulk = inf)."""
+    print(etype, flush=True)
+    coords, conn = meshgen.rect_tris(3, 3) if etype == cabi.TRIAG2D else meshgen.box_tetras(2, 2, 2)
+    case = case_of(etype, coords, conn)
+    case.u0 *= 1e160
+    d, k, X = case.dim, case.dim + 1, case.coords[case.conn]
+    start, _, slots = oracle.build_sparsity(case.conn, case.n_nodes)
+    grad = np.linalg.inv(X[:, 1:] - X[:, :1]).transpose(0, 2, 1)
+    grad = np.concatenate([-grad.sum(1, keepdims=True), grad], axis=1)
+    vol = np.abs(np.linalg.det(X[:, 1:] - X[:, :1])) / (2 if d == 2 else 6)
+    div = (vol / k)[:, None, None] * grad
+    ref = np.zeros((int(start[-1]), k))
+    np.add.at(ref[:, :d], slots.reshape(-1, k, k), np.broadcast_to(div[:, None], (len(div), k, k, d)))
+    rref = np.zeros(case.n_nodes)
+    np.add.at(rref, case.conn, -np.einsum("ebi,ebi->e", div, case.u0[case.conn])[:, None])
+    g = gpu_case(ctx, case, theta=0.7)
+    g.assemble(cabi.FP64)
+    v, r = g.system.values().reshape(-1, k, k)[:, d], g.system.vector(cabi.RHS).reshape(-1, k)[:, d]
+    assert np.abs(v - ref).max() <= 1e-12 * np.abs(ref).max()
+    assert np.abs(r - rref).max() <= 1e-12 * np.abs(rref).max()
+    g.close()
