@@ -124,7 +124,7 @@ __global__ void k_inc_from_keys(const uint64_t* __restrict__ keys, uint64_t nek,
   inc[t] = (uint32_t)(keys[t] % nek);
 }
 
-// contribution key: slot * 2^16 + b * 2^12 + q
+// contribution key: slot * 2^16 + b * 2^12 + q (a row with more incidences than q has bits is refused below)
 __global__ void k_contrib_keys(const uint32_t* __restrict__ conn, const uint32_t* __restrict__ inc,
                                const uint32_t* __restrict__ inc_ptr, const uint32_t* __restrict__ slots,
                                uint64_t nek, int k, uint64_t* __restrict__ keys)
@@ -133,7 +133,7 @@ __global__ void k_contrib_keys(const uint32_t* __restrict__ conn, const uint32_t
   if(t >= nek) return;
   const uint32_t ea = inc[t];
   const uint32_t row = conn[ea];
-  const uint32_t q = (uint32_t)(t - inc_ptr[row]);
+  const uint32_t q = min((uint32_t)(t - inc_ptr[row]), 4095u);
   for(int b = 0; b < k; ++b) {
     const uint64_t s = slots[(uint64_t)ea * k + b];
     keys[t * k + b] = (s << 16) | ((uint64_t)b << 12) | q;
@@ -202,7 +202,8 @@ __global__ void k_block_acc(uint64_t n_blocks, int passes, const uint32_t* __res
 }
 
 // Per row: accumulator threads of the staged reduction (low half) and block lists (high half; simplices,
-// len > 0), each saturated at 0xffff (above any workgroup's limit).
+// len > 0), each saturated at 0xffff (above any workgroup's limit).  A row of more incidences than a workgroup
+// holds is refused by the caller: its lists are not counted.
 __global__ void k_row_acc(uint32_t n, const uint32_t* __restrict__ row_ptr, const uint8_t* __restrict__ acc_cnt,
                           uint32_t len, bool periodic, int k, const uint32_t* __restrict__ contrib_ptr,
                           const uint16_t* __restrict__ contrib, const uint32_t* __restrict__ inc_ptr,
@@ -212,9 +213,10 @@ __global__ void k_row_acc(uint32_t n, const uint32_t* __restrict__ row_ptr, cons
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if(i >= n) return;
   uint32_t a = 0, l = 0;
+  const bool count = len > 0 && inc_ptr[i + 1] - inc_ptr[i] <= (uint32_t)kAsmThreads;
   for(uint32_t s = row_ptr[i]; s < row_ptr[i + 1]; ++s) {
     a += acc_cnt[s];
-    if(len == 0) continue;
+    if(!count) continue;
     const uint32_t c0 = contrib_ptr[s], nc = contrib_ptr[s + 1] - c0;
     if(!periodic) l += (nc + len - 1) / len;
     else for_block_lists(contrib + c0, nc, true, k, len, inc + inc_ptr[i], conn, [&](auto, uint32_t) { ++l; });

@@ -5,6 +5,8 @@ mesh nodes that hold different states.
 
 Bars: FP64 row-relative 1e-12 as everywhere; FP32 1e-6 of the element matrices plus one rounding per summed
 contribution."""
+import time
+
 import numpy as np
 import pytest
 
@@ -115,3 +117,20 @@ def test_infinite_tau_argument(ctx, oracle, etype):
     assert np.abs(v - ref).max() <= 1e-12 * np.abs(ref).max()
     assert np.abs(r - rref).max() <= 1e-12 * np.abs(rref).max()
     g.close()
+
+
+@pytest.mark.parametrize("n", [129, 5000, 70000])
+def test_periodic_hub_is_refused(ctx, n):
+    """All nodes of a ring linked to one: a block row of 2 n incidences and n column nodes, far above what a
+    workgroup holds (and, at n = 5000 and 70000, above the 12 bits of an incidence number in the contribution
+    lists), is refused at once."""
+    print(n, flush=True)
+    case = triangle_fan(n)
+    links = np.ones(n + 1, np.uint32)
+    active = (np.arange(n + 1) > 1).astype(np.uint8)
+    mesh = cabi.Mesh(ctx, case.etype, case.coords, case.conn)
+    t = time.perf_counter()
+    with pytest.raises(cabi.Cf3HipError, match="incident elements"):
+        cabi.System(ctx, mesh, periodic=(links, active))
+    assert time.perf_counter() - t < 2
+    mesh.close()
