@@ -200,17 +200,19 @@ __global__ void k_spmv_generic(uint32_t N, int neq, const uint32_t* __restrict__
 // (rhs[m, j] -= A[(m, j), (n, e)] * v_first(n, e); A[(m, j), (n, e)] = 0).  16 lanes per row, a lane the blocks
 // 16 apart: most rows have no such column and end after one round of mask bytes; one thread per row walked
 // its columns and masks one after the other (64^3 cube 156 us, now 64).
+// The workgroups walk the rows: one per 16 rows would exceed the 2^32 work-items of a launch beyond 2^28 rows.
+constexpr unsigned kColumnGrid = 1u << 22;
 template<typename T>
 __global__ __launch_bounds__(256) void k_dirichlet_columns(uint32_t N, int neq, const uint32_t* __restrict__ row_ptr,
                                                            const uint32_t* __restrict__ cols, T* __restrict__ vals,
                                                            const uint8_t* __restrict__ mask,
                                                            const double* __restrict__ vfirst, double* __restrict__ rhs)
 {
-  const uint32_t m = (blockIdx.x * 256 + threadIdx.x) >> 4, l = threadIdx.x & 15;
+  const uint32_t l = threadIdx.x & 15;
   const int nn = neq * neq;
-  double r[4] = {0., 0., 0., 0.};
-  bool touched = false;
-  if(m < N)
+  for(uint64_t m = (uint64_t)blockIdx.x * 16 + (threadIdx.x >> 4); m < N; m += (uint64_t)gridDim.x * 16) {
+    double r[4] = {0., 0., 0., 0.};
+    bool touched = false;
     for(uint32_t q = row_ptr[m] + l; q < row_ptr[m + 1]; q += 16) {
       const uint32_t n = cols[q];
       const uint8_t mk = mask[n];
@@ -228,13 +230,14 @@ __global__ __launch_bounds__(256) void k_dirichlet_columns(uint32_t N, int neq, 
           }
       }
     }
-  if(!rhs || !((__ballot(touched) >> (threadIdx.x & 48)) & 0xffffu)) return;   // whole 16-lane groups
+    if(!rhs || !((__ballot(touched) >> (threadIdx.x & 48)) & 0xffffu)) continue;   // whole 16-lane groups
 #pragma unroll
-  for(int j = 0; j < 4; ++j) r[j] = lanes::sum16(r[j]);
-  if(l == 0)
+    for(int j = 0; j < 4; ++j) r[j] = lanes::sum16(r[j]);
+    if(l == 0)
 #pragma unroll
-    for(int j = 0; j < 4; ++j)
-      if(j < neq) rhs[(uint64_t)m * neq + j] += r[j];
+      for(int j = 0; j < 4; ++j)
+        if(j < neq) rhs[m * neq + j] += r[j];
+  }
 }
 
 // symmetric Dirichlet, row part: BC row -> identity; rhs = sol = last value
@@ -722,7 +725,7 @@ void lss_dirichlet(Lss& L, uint32_t nbc, const uint32_t* nodes, const uint32_t* 
   if(nf)
     hipLaunchKernelGGL(k_scatter_conditions, dim3(grid_for(nf, 256)), dim3(256), 0, c.stream, nf, neq, dd + before,
                        dv + nall, L.bc_vfirst.as<double>(), L.bc_newmask.as<uint32_t>(), L.bc_mask.as<uint32_t>());
-  const dim3 gcol(grid_for((uint64_t)L.n_nodes * 16, 256));
+  const dim3 gcol(std::min<unsigned>(grid_for(L.n_nodes, 16), kColumnGrid));
   if(nf)
     hipLaunchKernelGGL(k_dirichlet_columns<double>, gcol, dim3(256), 0, c.stream, L.n_nodes, neq, L.row_ptr.as<uint32_t>(),
                        L.cols.as<uint32_t>(), L.values.as<double>(), L.bc_newmask.as<uint8_t>(),

@@ -4,6 +4,8 @@ node or one of them, and a reset in between.
 
 Bar: values exactly (entries are kept, zeroed or set to 1); rhs within (blocks of a row x neq + 2) eps of the
 sum of the absolute terms, whose order is the kernel's own."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -56,5 +58,32 @@ def test_conditions_against_oracle(oracle, neq, N):
             bar = (np.diff(start.astype(np.int64)).max() * neq + 2) * 2.0 ** -52 * scale
             assert (np.abs(s.vector(cabi.RHS) - rhs) <= bar).all()
     assert n == s.n_blocks
+    s.close()
+    ctx.close()
+
+
+def test_more_rows_than_lanes_in_32_bits():
+    """A condition that a row past 2^28 couples to (16 lanes per row: more than 2^32 lanes): identities but for the
+    last row, which holds the column of the one before it."""
+    N = 2 ** 28 + 5
+    start = np.arange(N + 1, dtype=np.uint32)
+    start[N] += 1
+    cols = np.arange(N + 1, dtype=np.uint32)
+    cols[N - 1], cols[N] = N - 2, N - 1
+    ctx = cabi.Context(0)
+    s = cabi.System(ctx, neq=1, graph=(start, cols, N))
+    del start, cols
+    s.reset(2.0)
+    s.reset_vector(cabi.RHS, 1.0)
+    print("system made", flush=True)
+    s.dirichlet([N - 2], [0], [3.0])
+    value = C.c_double()
+
+    def rhs(row):
+        cabi.check(cabi.lib().cf3hip_vector_get_value(s.h, cabi.RHS, row, 0, C.byref(value)))
+        return value.value
+    assert s.get_value(N - 2, N - 1) == 0.0 and rhs(N - 1) == 1.0 - 2.0 * 3.0
+    assert s.get_value(N - 2, N - 2) == 1.0 and rhs(N - 2) == 3.0
+    assert s.get_value(0, 0) == 2.0 and rhs(0) == 1.0
     s.close()
     ctx.close()
