@@ -120,12 +120,13 @@ __global__ void k_spmv_mixed_generic(uint32_t N, int neq, const uint32_t* __rest
 // to LDS as they are; one thread per scalar row then sums its own by fused multiply-adds, blocks and columns in
 // ascending order: bit for bit the sums of k_spmv_generic.  A range of more than stream_blocks blocks is taken
 // in pieces.  Bound by the value stream where enough workgroups fit into LDS: 512 x 512 quadrilaterals, neq = 3,
-// 180 MB, one thread per scalar row 93 us; 24 rows and 256 blocks (24 KB) 51 us, 216 blocks 46.7, 14 rows and 128
-// blocks 42 us (4.6 TB/s); 500^2 x 2 triangles 37.4 / 34.1 / 35.6.  FP32 (34.7 against 37.7 us) keeps the large ones.
-template<typename T> constexpr int stream_rows() { return sizeof(T) == 8 ? 14 : 24; }   // x 9 blocks of a quadrilateral mesh
-template<typename T> constexpr int stream_blocks() { return sizeof(T) == 8 ? 128 : 256; }
+// 180 MB, one thread per scalar row 93 us; 24 rows and 256 blocks (24 KB) 51 us, 24 and 216 46.7, 18 and 162 39.6
+// (4.9 TB/s), 14 and 128 42.1; 500^2 x 2 triangles 37.4 / 34.1 / 33.2 / 35.8.  FP32, 24 and 256: 34.7 (14 rows 37.7).
+template<typename T> constexpr int stream_rows() { return sizeof(T) == 8 ? 18 : 24; }   // x 9 blocks of a quadrilateral mesh
+template<typename T> constexpr int stream_blocks() { return sizeof(T) == 8 ? 162 : 256; }
+constexpr uint32_t kStreamGrid = 1u << 22;   // workgroups of one launch (of at most 2^32 work-items)
 template<typename T, typename VR, int NEQ>
-__global__ __launch_bounds__(256) void k_spmv_stream(uint32_t N, const uint32_t* __restrict__ row_ptr,
+__global__ __launch_bounds__(256) void k_spmv_stream(uint32_t base, uint32_t N, const uint32_t* __restrict__ row_ptr,
                                                      const uint32_t* __restrict__ cols, const VR* __restrict__ vals,
                                                      T alpha, const T* __restrict__ x, T beta, T* __restrict__ y,
                                                      const double* __restrict__ stop)
@@ -136,7 +137,7 @@ __global__ __launch_bounds__(256) void k_spmv_stream(uint32_t N, const uint32_t*
   __shared__ T s_x[BLOCKS * NEQ];
   if(stop && stop[0] != 0.) return;
   const uint32_t t = threadIdx.x;
-  const uint32_t row0 = blockIdx.x * ROWS;
+  const uint32_t row0 = base + blockIdx.x * ROWS;
   const uint32_t nr = min((uint32_t)ROWS, N - row0);
   const uint32_t b0 = row_ptr[row0], b1 = row_ptr[row0 + nr];
   const bool owner = t < nr * NEQ;
@@ -337,18 +338,24 @@ void lss_fill32(Context& c, float* p, size_t n, float v)
 }
 
 namespace {
+// (the pieces of a row range must not step past 2^32 blocks)
+bool streams(const Lss& L) { return (L.neq == 2 || L.neq == 3) && L.n_blocks < 0xffffff00ull; }
+
 template<typename T, typename VR>
 void spmv_stream(Lss& L, const VR* vals, T alpha, const T* x, T beta, T* y, const double* stop)
 {
-  const dim3 g(grid_for(L.n_nodes, stream_rows<T>()));
   const uint32_t* rp = L.row_ptr.as<uint32_t>();
   const uint32_t* cl = L.cols.as<uint32_t>();
-  if(L.neq == 2)
-    hipLaunchKernelGGL((k_spmv_stream<T, VR, 2>), g, dim3(256), 0, L.ctx->stream, L.n_nodes, rp, cl, vals, alpha, x, beta,
-                       y, stop);
-  else
-    hipLaunchKernelGGL((k_spmv_stream<T, VR, 3>), g, dim3(256), 0, L.ctx->stream, L.n_nodes, rp, cl, vals, alpha, x, beta,
-                       y, stop);
+  constexpr uint32_t ROWS = stream_rows<T>();
+  for(uint64_t base = 0; base < L.n_nodes; base += (uint64_t)ROWS * kStreamGrid) {
+    const dim3 g((unsigned)std::min<uint64_t>((L.n_nodes - base + ROWS - 1) / ROWS, kStreamGrid));
+    if(L.neq == 2)
+      hipLaunchKernelGGL((k_spmv_stream<T, VR, 2>), g, dim3(256), 0, L.ctx->stream, (uint32_t)base, L.n_nodes, rp, cl,
+                         vals, alpha, x, beta, y, stop);
+    else
+      hipLaunchKernelGGL((k_spmv_stream<T, VR, 3>), g, dim3(256), 0, L.ctx->stream, (uint32_t)base, L.n_nodes, rp, cl,
+                         vals, alpha, x, beta, y, stop);
+  }
 }
 }  // namespace
 
@@ -359,7 +366,7 @@ void lss_spmv(Lss& L, double alpha, const double* x, double beta, double* y, con
   if(L.neq == 4) {
     hipLaunchKernelGGL(k_spmv4_f64, dim3(grid_for((uint64_t)L.n_nodes * 16, 256)), dim3(256), 0, c.stream, L.n_nodes,
                        L.row_ptr.as<uint32_t>(), L.cols.as<uint32_t>(), L.values.as<double>(), alpha, x, beta, y, stop);
-  } else if(L.neq == 2 || L.neq == 3) {
+  } else if(streams(L)) {
     spmv_stream<double, double>(L, L.values.as<double>(), alpha, x, beta, y, stop);
   } else {
     hipLaunchKernelGGL(k_spmv_generic<double>, dim3(grid_for(L.dofs, 256)), dim3(256), 0, c.stream, L.n_nodes, L.neq,
@@ -378,7 +385,7 @@ void lss_spmv32(Lss& L, float alpha, const float* x, float beta, float* y, const
   if(L.neq == 4) {
     hipLaunchKernelGGL(k_spmv4_f32, dim3(grid_for((uint64_t)L.n_nodes * 16, 256)), dim3(256), 0, c.stream, L.n_nodes,
                        L.row_ptr.as<uint32_t>(), L.cols.as<uint32_t>(), L.values32.as<float>(), alpha, x, beta, y, stop);
-  } else if(L.neq == 2 || L.neq == 3) {
+  } else if(streams(L)) {
     spmv_stream<float, float>(L, L.values32.as<float>(), alpha, x, beta, y, stop);
   } else {
     hipLaunchKernelGGL(k_spmv_generic<float>, dim3(grid_for(L.dofs, 256)), dim3(256), 0, c.stream, L.n_nodes, L.neq,
@@ -397,7 +404,7 @@ void lss_spmv_mixed(Lss& L, const double* x, double* y, const double* stop)
   if(L.neq == 4) {
     hipLaunchKernelGGL(k_spmv4_mixed, dim3(grid_for((uint64_t)L.n_nodes * 16, 256)), dim3(256), 0, c.stream, L.n_nodes,
                        L.row_ptr.as<uint32_t>(), L.cols.as<uint32_t>(), L.values32.as<float>(), x, y, stop);
-  } else if(L.neq == 2 || L.neq == 3) {
+  } else if(streams(L)) {
     spmv_stream<double, float>(L, L.values32.as<float>(), 1., x, 0., y, stop);
   } else {
     hipLaunchKernelGGL(k_spmv_mixed_generic, dim3(grid_for(L.dofs, 256)), dim3(256), 0, c.stream, L.n_nodes, L.neq,

@@ -3,6 +3,8 @@
 shorter and longer than one trip of loads), beside 1 equation per node.
 
 Bar: every entry within (terms + 3) eps of the dot product of absolute values, eps of the arithmetic."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -20,7 +22,7 @@ def graph(N, seed):
 
 
 @pytest.mark.parametrize("neq", [1, 2, 3, 4])
-@pytest.mark.parametrize("N", [1, 23, 24, 25, 301])
+@pytest.mark.parametrize("N", [1, 17, 18, 19, 23, 24, 25, 301])
 def test_product_on_ragged_rows(neq, N):
     start, cols = graph(N, 10 * N + neq)
     rng = np.random.default_rng(N)
@@ -94,5 +96,24 @@ def test_products_are_fused(neq):
             s.apply_fp32_device(1.0, s.vector_ptr(cabi.SOLUTION), 0.0, s.vector_ptr(cabi.RHS))
             y = s.vector(cabi.RHS).view(np.float32)[:N * neq]
         assert (y == e * e).all()
+    s.close()
+    ctx.close()
+
+
+def test_product_of_more_rows_than_workgroups():
+    """Diagonal blocks in more rows than 2^32 work-items serve: the last rows are multiplied too."""
+    N = 2 ** 28 + 3
+    ctx = cabi.Context(0)
+    s = cabi.System(ctx, neq=2, graph=(np.arange(N + 1, dtype=np.uint32), np.arange(N, dtype=np.uint32), N))
+    s.reset(0.5)
+    s.reset_vector(cabi.SOLUTION, 3.0)
+    s.reset_vector(cabi.RHS, 1.0)
+    print("system made", flush=True)
+    s.apply_device(2.0, s.vector_ptr(cabi.SOLUTION), 1.0, s.vector_ptr(cabi.RHS))
+    value = C.c_double()
+    for row in (0, 2 ** 22 * 18 - 1, 2 ** 22 * 18, N // 2, N - 2, N - 1):   # 18 rows a workgroup
+        for eq in (0, 1):
+            cabi.check(cabi.lib().cf3hip_vector_get_value(s.h, cabi.RHS, row, eq, C.byref(value)))
+            assert value.value == 2.0 * (0.5 * 3.0 + 0.5 * 3.0) + 1.0, (row, eq)
     s.close()
     ctx.close()
