@@ -298,10 +298,12 @@ inline uint32_t plan_segment(uint64_t rows) { return rows < 65536 ? 63 : 252; }
 
 // Distance in rows from each incidence's row back to the nearest earlier row of its element (255: none
 // within 254): the element is new to a workgroup that starts at r0 exactly when that row is before r0.
+// Clears info[5], which the following kernels fill.
 __global__ void k_inc_back(uint64_t nek, int k, const uint32_t* __restrict__ inc, const uint32_t* __restrict__ rconn,
-                           uint8_t* __restrict__ back)
+                           uint8_t* __restrict__ back, uint32_t* __restrict__ info)
 {
   const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if(t < 5) info[t] = 0;
   if(t >= nek) return;
   const uint32_t ea = inc[t], a = ea % (uint32_t)k;
   const uint32_t* en = rconn + (ea - a);
@@ -315,7 +317,7 @@ __global__ void k_inc_back(uint64_t nek, int k, const uint32_t* __restrict__ inc
   back[t] = (uint8_t)d;
 }
 
-// One wave per segment of rows: start[r] = 1 where a workgroup starts.  fits stays 0 unless a row alone
+// One wave per segment of rows: start[r] = 1 where a workgroup starts.  misfit becomes 1 when a row alone
 // exceeds a limit.
 __global__ __launch_bounds__(64) void k_plan_partition(uint32_t N, uint32_t segment, const uint32_t* __restrict__ inc_ptr,
                                                        const uint8_t* __restrict__ back,
@@ -343,12 +345,6 @@ __global__ __launch_bounds__(64) void k_plan_partition(uint32_t N, uint32_t segm
     else { ne += fresh; nl += lists; }
     if(lane == 0) start[r] = open ? 1 : 0;
   }
-}
-
-__global__ void k_iota(uint32_t n, uint32_t* __restrict__ out)
-{
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if(i < n) out[i] = i;
 }
 
 // ascending bitonic sort of S (a power of two) LDS values
@@ -689,7 +685,9 @@ void build_element_structures(Lss& L)
     HIP_OK(hipGetLastError());
   }
   // accumulator threads per block and per row
-  const uint32_t list_len = q1 ? 0 : plan_list_length((int)k);
+  // (block lists: the specialised simplex kernels, which take systems of dim + 1 equations only)
+  const bool plans = !q1 && L.neq == M.dim + 1;
+  const uint32_t list_len = plans ? plan_list_length((int)k) : 0;
   acc_cnt.alloc(&c, L.n_blocks);
   row_acc.alloc(&c, sizeof(uint32_t) * N);
   hipLaunchKernelGGL(k_block_acc, dim3(grid_for(L.n_blocks, 256)), dim3(256), 0, c.stream, L.n_blocks, L.passes,
@@ -746,30 +744,28 @@ void build_element_structures(Lss& L)
                      L.inc_pos.as<uint8_t>(), L.blk_beg.as<uint8_t>(), L.blk_acc.as<uint16_t>());
   HIP_OK(hipGetLastError());
 
-  // ---- assembly plans (simplices) ----
-  if(!q1 && N > 0) {
-    // one allocation: info (n_plan, misfit, most[3]), row numbers, workgroup starts, start flags, back
-    DevBuf scratch, temp;
-    scratch.alloc(&c, 32 + 9 * N + nek);
+  // ---- assembly plans (specialised simplices) ----
+  if(plans && N > 0) {
+    // one allocation: info (n_plan, misfit, most[3]), workgroup starts, start flags, back, room of the selection
+    const hipcub::CountingInputIterator<uint32_t> rows(0);
+    size_t temp_bytes = 0;
+    HIP_OK(hipcub::DeviceSelect::Flagged(nullptr, temp_bytes, rows, (uint8_t*)nullptr, (uint32_t*)nullptr,
+                                         (uint32_t*)nullptr, (int)N, c.stream));
+    const size_t head = (32 + 5 * N + nek + 255) / 256 * 256;
+    DevBuf scratch;
+    scratch.alloc(&c, head + std::max<size_t>(temp_bytes, 16));
     uint32_t* inf = scratch.as<uint32_t>();
-    uint32_t *rows = inf + 8, *starts = rows + N;
+    uint32_t* starts = inf + 8;
     uint8_t* flag = reinterpret_cast<uint8_t*>(starts + N);
     uint8_t* back = flag + N;
-    uint32_t host[5] = {0, 0, 0, 0, 0};
-    HIP_OK(hipMemcpyAsync(inf, host, sizeof(host), hipMemcpyHostToDevice, c.stream));
+    uint32_t host[5];
     hipLaunchKernelGGL(k_inc_back, dim3(grid_for(nek, 256)), dim3(256), 0, c.stream, nek, (int)k, L.inc.as<uint32_t>(),
-                       conn, back);
+                       conn, back, inf);
     hipLaunchKernelGGL(k_plan_partition, dim3(grid_for(N, plan_segment(N))), dim3(64), 0, c.stream, (uint32_t)N,
-                       plan_segment(N),
-                       L.inc_ptr.as<uint32_t>(), back, row_acc.as<uint32_t>(), flag,
+                       plan_segment(N), L.inc_ptr.as<uint32_t>(), back, row_acc.as<uint32_t>(), flag,
                        reinterpret_cast<int*>(inf + 1));
-    hipLaunchKernelGGL(k_iota, dim3(grid_for(N, 256)), dim3(256), 0, c.stream, (uint32_t)N, rows);
-    size_t temp_bytes = 0;
-    HIP_OK(hipcub::DeviceSelect::Flagged(nullptr, temp_bytes, rows, flag,
-                                         starts, inf, (int)N, c.stream));
-    temp.alloc(&c, std::max<size_t>(temp_bytes, 16));
-    HIP_OK(hipcub::DeviceSelect::Flagged(temp.ptr, temp_bytes, rows, flag,
-                                         starts, inf, (int)N, c.stream));
+    HIP_OK(hipcub::DeviceSelect::Flagged(scratch.as<char>() + head, temp_bytes, rows, flag, starts, inf, (int)N,
+                                         c.stream));
     HIP_OK(hipMemcpyAsync(host, inf, sizeof(host), hipMemcpyDeviceToHost, c.stream));
     HIP_OK(hipStreamSynchronize(c.stream));
     const uint32_t n_plan = host[0];

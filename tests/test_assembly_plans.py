@@ -134,3 +134,21 @@ def test_periodic_hub_is_refused(ctx, n):
         cabi.System(ctx, mesh, periodic=(links, active))
     assert time.perf_counter() - t < 2
     mesh.close()
+
+
+def test_plans_only_where_they_are_read(ctx):
+    """The specialised kernels take dim + 1 equations: systems of other sizes hold no plans (about 100 bytes a node
+    of a triangle mesh, 350 of tetrahedra)."""
+    for coords, conn, etype, least in ((*meshgen.rect_tris(24, 24), cabi.TRIAG2D, 60),
+                                       (*meshgen.box_tetras(8, 8, 8), cabi.TETRA3D, 200)):
+        mesh = cabi.Mesh(ctx, etype, coords, conn)
+        N, full = len(coords), coords.shape[1] + 1
+        extra = {}
+        for neq in (1, 2, full):
+            before = ctx.memory()
+            s = cabi.System(ctx, mesh, neq=neq)
+            extra[neq] = ctx.memory() - before - 8 * (s.n_blocks * neq * neq + 2 * N * neq)
+            s.close()
+        print(N, extra, flush=True)
+        assert extra[1] == extra[2] and extra[full] >= extra[1] + least * N
+        mesh.close()
