@@ -743,7 +743,7 @@ struct PlanLayout {
   // record stride: an odd number of 16-byte pieces, so that the records spread over the banks
   static constexpr int STRIDE = (((WORDS * (int)sizeof(R) + 15) / 16) | 1) * 16 / (int)sizeof(R);
   static constexpr int LDW = D == 3 ? lds_row<R, NN>() : NN;   // 9 values: odd by themselves
-  static size_t lds_bytes(bool rhs, uint32_t nodes, uint32_t elems, uint32_t lists)
+  static constexpr size_t lds_bytes(bool rhs, uint32_t nodes, uint32_t elems, uint32_t lists)
   {
     const size_t stage = (size_t)nodes * (rhs ? 56 : 88);
     const size_t rec = sizeof(R) * STRIDE * (elems + 1);
@@ -1195,8 +1195,8 @@ void launch(const AsmArgs& g, const Lss& L)
   timer_end(c, CF3HIP_KERNEL_ASSEMBLY);
 }
 
-// specialised simplices: by block lists; a system without plans (a workgroup that touches more than
-// kPlanNodes nodes, or a node with too many elements) takes the staged reduction
+// specialised simplices: by block lists; a system without plans (a row of more elements or block lists than a
+// plan holds) takes the staged reduction
 template<int D, typename R, bool RHS>
 void launch_spec(const AsmArgs& g, const Lss& L, Fields& F)
 {
@@ -1358,6 +1358,8 @@ namespace {
 constexpr unsigned kBatchPackGrid = 1024;
 constexpr unsigned kBatchAsmGrid = 2048;   // persistent workgroups (8 per CU)
 constexpr size_t kBatchHeaderBytes = 256;
+constexpr size_t kBatchLds = 16384;   // of the captured assembly launch, enough for any plan
+static_assert(PlanLayout<3, float>::lds_bytes(false, kPlanNodes, kPlanElems, kAsmThreads) <= kBatchLds);
 }  // namespace
 
 size_t batch_table_bytes(uint32_t max_cases) { return kBatchHeaderBytes + sizeof(BatchEntry) * max_cases; }
@@ -1368,7 +1370,6 @@ void batch_assemble(Batch& B, uint32_t n, Lss* const* L, Fields* const* F, const
   BatchHeader* hd = reinterpret_cast<BatchHeader*>(B.host_table);
   BatchEntry* ent = reinterpret_cast<BatchEntry*>(static_cast<char*>(B.host_table) + kBatchHeaderBytes);
   uint32_t wg = 0, nodes = 0;
-  size_t lds = 16384;   // LDS of the captured launch; systems that need more capture it again
   for(uint32_t i = 0; i < n; ++i) {
     Lss& Li = *L[i];
     Fields& Fi = *F[i];
@@ -1401,29 +1402,20 @@ void batch_assemble(Batch& B, uint32_t n, Lss* const* L, Fields* const* F, const
     ent[i].n_nodes = Li.n_nodes;
     wg += Li.n_plan;
     nodes += Li.n_nodes;
-    if(Li.n_plan)
-      lds = std::max(lds, PlanLayout<3, float>::lds_bytes(false, Li.plan_nodes, Li.plan_elems, Li.plan_lists));
   }
   hd->n_cases = n;
   hd->total_wg = n ? wg : 0;
   hd->total_nodes = n ? nodes : 0;
   HIP_OK(hipMemcpyAsync(B.table.ptr, B.host_table, kBatchHeaderBytes + sizeof(BatchEntry) * (n ? n : 1),
                         hipMemcpyHostToDevice, B.stream));
-  if(B.exec && lds > B.lds) {
-    HIP_OK(hipGraphExecDestroy(B.exec));
-    HIP_OK(hipGraphDestroy(B.graph));
-    B.exec = nullptr;
-    B.graph = nullptr;
-  }
   if(!B.exec) {
-    B.lds = lds;
     // the two launches read the table from device memory, so one capture serves every later batch
     const BatchHeader* dh = B.table.as<BatchHeader>();
     const BatchEntry* de = reinterpret_cast<const BatchEntry*>(B.table.as<char>() + kBatchHeaderBytes);
     hipGraph_t graph = nullptr;
     HIP_OK(hipStreamBeginCapture(B.stream, hipStreamCaptureModeThreadLocal));
     hipLaunchKernelGGL(k_batch_pack, dim3(kBatchPackGrid), dim3(256), 0, B.stream, dh, de);
-    hipLaunchKernelGGL(k_batch_assemble, dim3(kBatchAsmGrid), dim3(kThreads), lds, B.stream, dh, de);
+    hipLaunchKernelGGL(k_batch_assemble, dim3(kBatchAsmGrid), dim3(kThreads), kBatchLds, B.stream, dh, de);
     HIP_OK(hipStreamEndCapture(B.stream, &graph));
     HIP_OK(hipGraphInstantiate(&B.exec, graph, nullptr, nullptr, 0));
     B.graph = graph;

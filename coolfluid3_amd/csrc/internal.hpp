@@ -92,8 +92,10 @@ constexpr int kMaxRedBlocks = 1024;
 // (one owner thread per block); the row schedule of the system respects both
 constexpr int kAsmThreads = 128;
 // Assembly plans of the specialised simplex kernels (see sparsity.hip).  A workgroup holds at most
-// kPlanElems elements (its record kPlanElems stands for none), kAsmThreads block lists and kPlanNodes nodes.
-constexpr uint32_t kPlanElems = 127, kPlanNodes = 255;
+// kPlanElems elements (its record kPlanElems stands for none) and kAsmThreads block lists, and so at most
+// kPlanNodes nodes: each node of an element is the column of a block of the row that holds the element there,
+// and a list has one column node.
+constexpr uint32_t kPlanElems = 127, kPlanNodes = kAsmThreads;
 constexpr uint32_t plan_list_length(int k) { return k == 4 ? 6 : 3; }   // contributions per block list, at most
 constexpr uint32_t kPlanHeadBytes = 32;                                  // r0, rows, elements, nodes, blk0, blocks, lists, 0
 constexpr uint32_t plan_bytes(uint32_t ns) { return kPlanHeadBytes + 4 * ns + kAsmThreads * (4 + 8 + 2); }
@@ -256,7 +258,6 @@ struct Batch {
   void* host_table = nullptr;   // pinned mirror
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
-  size_t lds = 0;               // dynamic LDS of the captured assembly launch
 };
 
 // ---------------------------------------------------------------------------------------------

@@ -422,8 +422,8 @@ __global__ __launch_bounds__(kAsmThreads) void k_plan_fill(uint32_t N, uint32_t 
                                                            const uint16_t* __restrict__ contrib,
                                                            unsigned char* __restrict__ plans, uint32_t* __restrict__ most)
 {
-  constexpr uint32_t S = kAsmThreads * 4;   // at least the nodes and the incidences of kPlanElems elements
-  __shared__ uint32_t s_etab[2 * kAsmThreads], s_ntab[2 * S], s_uniq[S], s_wave[kAsmThreads / 64];
+  constexpr uint32_t S = kAsmThreads * 4;   // at least the incidences of kPlanElems elements
+  __shared__ uint32_t s_etab[2 * kAsmThreads], s_ntab[2 * kPlanNodes], s_uniq[kPlanNodes], s_wave[kAsmThreads / 64];
   __shared__ uint32_t s_elem[kAsmThreads], s_loc[kAsmThreads];
   __shared__ uint8_t s_eidx[2 * kAsmThreads];
   __shared__ uint16_t s_inc[S];             // per incidence: element << 2 | a
@@ -433,7 +433,7 @@ __global__ __launch_bounds__(kAsmThreads) void k_plan_fill(uint32_t N, uint32_t 
   const uint32_t i0 = inc_ptr[r0], ninc = inc_ptr[r1] - i0;
   const uint32_t blk0 = row_ptr[r0], nblk = row_ptr[r1] - blk0;
   for(uint32_t j = t; j < 2 * kAsmThreads; j += kAsmThreads) s_etab[j] = 0xffffffffu;
-  for(uint32_t j = t; j < 2 * S; j += kAsmThreads) s_ntab[j] = 0xffffffffu;
+  for(uint32_t j = t; j < 2 * kPlanNodes; j += kAsmThreads) s_ntab[j] = 0xffffffffu;
   __syncthreads();
   // distinct elements, in the order of their first incidence
   uint32_t ne = 0;
@@ -454,23 +454,22 @@ __global__ __launch_bounds__(kAsmThreads) void k_plan_fill(uint32_t N, uint32_t 
     ne += total;
   }
   __syncthreads();
-  // distinct nodes, ascending
+  // distinct nodes, ascending (at most kPlanNodes: one list at least names each)
   uint32_t mine[4] = {0, 0, 0, 0}, f = 0, nn;
   if(t < ne)
     for(int m = 0; m < k; ++m) {
       bool put;
       mine[m] = conn[(uint64_t)s_elem[t] * k + m];
-      (void)lds_insert<2 * S>(s_ntab, mine[m], put);
+      (void)lds_insert<2 * kPlanNodes>(s_ntab, mine[m], put);
       f |= put ? 1u << m : 0u;
     }
   uint32_t o = wg_scan((uint32_t)__popc(f), s_wave, t, nn);
-  for(uint32_t j = t; j < S; j += kAsmThreads) s_uniq[j] = 0xffffffffu;
+  for(uint32_t j = t; j < kPlanNodes; j += kAsmThreads) s_uniq[j] = 0xffffffffu;
   __syncthreads();
   for(int m = 0; m < 4; ++m)
     if(f & (1u << m)) s_uniq[o++] = mine[m];
   __syncthreads();
-  if(nn <= kAsmThreads) lds_sort<kAsmThreads>(s_uniq, t);
-  else lds_sort<S>(s_uniq, t);
+  lds_sort<kPlanNodes>(s_uniq, t);
   uint32_t packed = 0;
   if(t < ne)
     for(int m = 0; m < k; ++m) packed |= lds_find(s_uniq, nn, mine[m]) << (8 * m);
@@ -592,7 +591,7 @@ void build_element_structures(Lss& L)
   const uint64_t N = L.n_nodes, E = M.n_elems, k = M.k;   // N block rows
   const uint64_t npairs = E * k * k, nek = E * k;
   // rows and columns of the element nodes (the mesh nodes, or their block rows under periodic links);
-  // the gathers of the kernels (and the node staging lists) keep the mesh nodes of M.conn
+  // the gathers of the kernels (and the nodes of the assembly plans) keep the mesh nodes of M.conn
   DevBuf dconn;
   const uint32_t* conn = M.conn.as<uint32_t>();
   if(L.periodic) {
@@ -787,8 +786,7 @@ void build_element_structures(Lss& L)
         break;
       }
       L.plan.release();
-      if(host[2] > kPlanNodes) break;
-      ns = (host[2] + 3) / 4 * 4;
+      ns = (host[2] + 3) / 4 * 4;   // at most kPlanNodes
     }
   }
   HIP_OK(hipStreamSynchronize(c.stream));

@@ -152,3 +152,30 @@ def test_plans_only_where_they_are_read(ctx):
         print(N, extra, flush=True)
         assert extra[1] == extra[2] and extra[full] >= extra[1] + least * N
         mesh.close()
+
+
+def test_batch_with_systems_beyond_the_plans(ctx):
+    """Systems with a row that no plan holds, in a batch with others (first, between, last, alone): every system
+    gets the bits of its own single assembly."""
+    def make(case):
+        g = gpu_case(ctx, case, fp32=True)
+        g.assemble(cabi.FP32)
+        return g, g.system.values_fp32()
+    hub = [make(tetrahedron_fan(97)) for _ in range(3)]
+    tets = [make(case_of(cabi.TETRA3D, *meshgen.box_tetras(n, n, n), seed=n)) for n in (3, 6)]
+    batch = cabi.Batch(ctx, 5)
+    for group in ([hub[0]] + tets, [tets[0], hub[0], tets[1]], tets + [hub[0]], [hub[0]], hub, [tets[1]],
+                  [hub[0], tets[0], hub[1], tets[1], hub[2]]):
+        print(len(group), flush=True)
+        for g, _ in group:
+            g.system.reset(7.0)
+            g.system.round_fp32()
+        prms = [cabi.NSParams.from_buffer_copy(g.prm) for g, _ in group]
+        for p in prms:
+            p.precision = cabi.FP32
+        batch.assemble([g.system for g, _ in group], [g.fields for g, _ in group], prms)
+        for g, ref in group:
+            assert np.array_equal(g.system.values_fp32(), ref)
+    batch.close()
+    for g, _ in hub + tets:
+        g.close()

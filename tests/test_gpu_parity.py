@@ -132,8 +132,8 @@ def quads_case(n=9, seed=11):
 
 def scattered_tets_case(n=512, seed=7):
     """Disjoint tetrahedra whose nodes are numbered a quarter of the mesh apart (tet k has nodes k,
-    k + n, k + 2n, k + 3n): a workgroup of 128 one-incidence rows touches 512 distinct nodes, above
-    the 255 of node staging, so the FP64 kernel runs unstaged on this mesh."""
+    k + n, k + 2n, k + 3n): consecutive rows share no element, so the block-list workgroups hold 32 rows of
+    four lists and 128 distinct nodes, the most there can be."""
     rng = np.random.default_rng(seed)
     base = rng.uniform(0.0, 10.0, (n, 3))
     unit = np.array([[0.0, 0.0, 0.0], [1.0, 0.0, 0.0], [0.0, 1.0, 0.0], [0.0, 0.0, 1.0]])

@@ -151,7 +151,7 @@ def test_periodic_system_refuses_the_matrix_free_forms():
 @pytest.mark.parametrize("name", ["tets", "hexas"])
 def test_periodic_3d_assembly_vs_oracle(name):
     """3D periodic links (x: right -> left, then y: back -> front) on the tetrahedral cube (specialised,
-    node-staged FP64 kernel) and the hexahedral cube (Q1 kernel): sparsity and slot map bit-exact
+    block-list FP64 kernel) and the hexahedral cube (Q1 kernel): sparsity and slot map bit-exact
     against the oracle's sparsity of p2m[conn], FP64 values and rhs within 1e-12."""
     o = pyoracle.get()
     # without jitter: the tangential jitter of the boundary nodes would break the periodic matching
