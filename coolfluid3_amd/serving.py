@@ -64,11 +64,14 @@ def device_bytes_estimate(cells):
     meshes) the FP64, FP32 and block-scaled FP32 values, its column and staging bytes; per element the
     connectivity, incidences, staging positions and element-to-slot map; per node the BiCGStab
     workspace (10 vectors), the FGMRES workspace of the fallback (35 vectors), D^-1, the fields, the
-    packed node records and the rhs / solution / residual vectors."""
+    packed node records, the rhs / solution / residual vectors, the assembly plans (2080 bytes for 5.2 to
+    6 rows) and the conditions' values and masks; per boundary node its share of the conditions' upload
+    (4 conditions of two values and a dof, with half as much room again)."""
     N = (cells + 1) ** 3
     E = 6 * cells ** 3
     nb = 15 * N
-    return nb * (128 + 64 + 64 + 4 + 6) + E * (16 + 16 + 16 + 64) + N * (320 + 1120 + 128 + 160 + 96 + 96 + 16)
+    return (nb * (128 + 64 + 64 + 4 + 6) + E * (16 + 16 + 16 + 64) + N * (320 + 1120 + 128 + 160 + 96 + 96 + 16 + 400 + 34) +
+            6 * (cells + 1) ** 2 * 120)
 
 
 class _Case:

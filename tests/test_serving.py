@@ -112,6 +112,16 @@ def test_continuous_progress_and_admission():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("cells", [4, 12, 28])
+def test_memory_estimate_covers_the_fallback(cells):
+    """The estimate is an upper one: it holds with the FGMRES workspace of the fallback (35 vectors) on top of what
+    an ordinary request ends with."""
+    recs, _ = serving.Server().run([serving.Request(0, 0.0, cells, 200.0, 0.05, steps=1)])
+    print(cells, recs[0].device_bytes, recs[0].bytes_estimate, flush=True)
+    assert recs[0].device_bytes + 35 * 4 * 8 * (cells + 1) ** 3 <= recs[0].bytes_estimate
+
+
+@pytest.mark.gpu
 @pytest.mark.timeout(900)
 def test_serving_stream_512():
     """The 512-request stream (Poisson arrivals at 200 req/s, cells log-uniform in [12, 64], Re in
