@@ -114,31 +114,43 @@ __global__ void k_spmv_mixed_generic(uint32_t N, int neq, const uint32_t* __rest
   y[r] = acc;
 }
 
-// neq = 2 or 3 (values VR, vectors T): a workgroup owns stream_rows node rows and streams their values as one
-// contiguous array, consecutive lanes on consecutive values (a block of 4 or 9 values is no multiple of a
-// 16-byte load, and one thread per scalar row reads it with a stride of a whole row).  Values and gathered x go
-// to LDS as they are; one thread per scalar row then sums its own by fused multiply-adds, blocks and columns in
-// ascending order: bit for bit the sums of k_spmv_generic.  A range of more than stream_blocks blocks is taken
-// in pieces.  Bound by the value stream where enough workgroups fit into LDS: 512 x 512 quadrilaterals, neq = 3,
-// 180 MB, one thread per scalar row 93 us; 24 rows and 256 blocks (24 KB) 51 us, 24 and 216 46.7, 18 and 162 39.6
-// (4.9 TB/s), 14 and 128 42.1; 500^2 x 2 triangles 37.4 / 34.1 / 33.2 / 35.8.  FP32, 24 and 256: 34.7 (14 rows 37.7).
-template<typename T> constexpr int stream_rows() { return sizeof(T) == 8 ? 18 : 24; }   // x 9 blocks of a quadrilateral mesh
-template<typename T> constexpr int stream_blocks() { return sizeof(T) == 8 ? 162 : 256; }
+// neq = 2 or 3 (values VR, vectors T): a workgroup owns some node rows and streams their values as one contiguous
+// array, consecutive lanes on consecutive values (a block of 4 or 9 values is no multiple of a 16-byte load, and
+// one thread per scalar row reads it with a stride of a whole row).  Values and gathered x go to LDS as they
+// are; one thread per scalar row then sums its own by fused multiply-adds, blocks and columns in ascending
+// order: bit for bit the sums of k_spmv_generic.  A range of more than stream_blocks blocks is taken in pieces.
+// Bound by the value stream where enough workgroups fit into LDS (12 to 16 KB each, rounded to what measured best):
+// 512 x 512 quadrilaterals, neq = 3, 180 MB, one thread per scalar row 75 us (FP32 58), 256 blocks 51, 216 46.7,
+// 162 39.3 (4.9 TB/s), 128 42.1; FP32 128 37.7, 256 32.0.  4 M blocks of neq = 2 in rows of 9: 70 us (64), 162 blocks 41.8,
+// 256 33.1, 288 35.8; FP32 256 29.4, 512 26.6.
+template<typename T>
+constexpr int stream_blocks(int neq) { return sizeof(T) == 8 ? (neq == 2 ? 256 : 162) : (neq == 2 ? 512 : 256); }
+// Rows of a workgroup: as many as fill stream_blocks on average, at most one thread per scalar row.  4 M blocks in rows
+// of 1, 3, 7, 15, 27, FP64 (FP32), us: neq = 3, one thread per scalar row 111, 146, 153, 183, 183 (69, 59, 88, 107, 124); 18
+// (24) rows 277, 119, 97, 96, 102 (170, 74, 54, 57, 65); this 115, 92, 90, 93, 93 (81, 51, 50, 50, 53).  neq = 2, a thread per
+// row 58, 43, 67, 82, 82; this 61, 37, 34, 34, 36.
+template<typename T>
+uint32_t stream_rows(const Lss& L)
+{
+  const uint64_t fill = (uint64_t)stream_blocks<T>(L.neq) * L.n_nodes / std::max<uint64_t>(L.n_blocks, 1);
+  return (uint32_t)std::min<uint64_t>(std::max<uint64_t>(fill, 1), 256 / L.neq);
+}
 constexpr uint32_t kStreamGrid = 1u << 22;   // workgroups of one launch (of at most 2^32 work-items)
 template<typename T, typename VR, int NEQ>
-__global__ __launch_bounds__(256) void k_spmv_stream(uint32_t base, uint32_t N, const uint32_t* __restrict__ row_ptr,
+__global__ __launch_bounds__(256) void k_spmv_stream(uint32_t base, uint32_t rows, uint32_t N,
+                                                     const uint32_t* __restrict__ row_ptr,
                                                      const uint32_t* __restrict__ cols, const VR* __restrict__ vals,
                                                      T alpha, const T* __restrict__ x, T beta, T* __restrict__ y,
                                                      const double* __restrict__ stop)
 {
-  constexpr int NN = NEQ * NEQ, ROWS = stream_rows<T>(), BLOCKS = stream_blocks<T>();
+  constexpr int NN = NEQ * NEQ, BLOCKS = stream_blocks<T>(NEQ);
   constexpr int TRIPS = (BLOCKS * NEQ + 255) / 256, VTRIPS = (BLOCKS * NN + 255) / 256;
   __shared__ VR s_val[BLOCKS * NN];
   __shared__ T s_x[BLOCKS * NEQ];
   if(stop && stop[0] != 0.) return;
   const uint32_t t = threadIdx.x;
-  const uint32_t row0 = base + blockIdx.x * ROWS;
-  const uint32_t nr = min((uint32_t)ROWS, N - row0);
+  const uint32_t row0 = base + blockIdx.x * rows;
+  const uint32_t nr = min(rows, N - row0);
   const uint32_t b0 = row_ptr[row0], b1 = row_ptr[row0 + nr];
   const bool owner = t < nr * NEQ;
   const uint32_t i = t / NEQ, a = t % NEQ;
@@ -346,15 +358,15 @@ void spmv_stream(Lss& L, const VR* vals, T alpha, const T* x, T beta, T* y, cons
 {
   const uint32_t* rp = L.row_ptr.as<uint32_t>();
   const uint32_t* cl = L.cols.as<uint32_t>();
-  constexpr uint32_t ROWS = stream_rows<T>();
-  for(uint64_t base = 0; base < L.n_nodes; base += (uint64_t)ROWS * kStreamGrid) {
-    const dim3 g((unsigned)std::min<uint64_t>((L.n_nodes - base + ROWS - 1) / ROWS, kStreamGrid));
+  const uint32_t rows = stream_rows<T>(L);
+  for(uint64_t base = 0; base < L.n_nodes; base += (uint64_t)rows * kStreamGrid) {
+    const dim3 g((unsigned)std::min<uint64_t>((L.n_nodes - base + rows - 1) / rows, kStreamGrid));
     if(L.neq == 2)
-      hipLaunchKernelGGL((k_spmv_stream<T, VR, 2>), g, dim3(256), 0, L.ctx->stream, (uint32_t)base, L.n_nodes, rp, cl,
-                         vals, alpha, x, beta, y, stop);
+      hipLaunchKernelGGL((k_spmv_stream<T, VR, 2>), g, dim3(256), 0, L.ctx->stream, (uint32_t)base, rows, L.n_nodes, rp,
+                         cl, vals, alpha, x, beta, y, stop);
     else
-      hipLaunchKernelGGL((k_spmv_stream<T, VR, 3>), g, dim3(256), 0, L.ctx->stream, (uint32_t)base, L.n_nodes, rp, cl,
-                         vals, alpha, x, beta, y, stop);
+      hipLaunchKernelGGL((k_spmv_stream<T, VR, 3>), g, dim3(256), 0, L.ctx->stream, (uint32_t)base, rows, L.n_nodes, rp,
+                         cl, vals, alpha, x, beta, y, stop);
   }
 }
 }  // namespace

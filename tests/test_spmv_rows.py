@@ -22,7 +22,7 @@ def graph(N, seed):
 
 
 @pytest.mark.parametrize("neq", [1, 2, 3, 4])
-@pytest.mark.parametrize("N", [1, 17, 18, 19, 23, 24, 25, 301])
+@pytest.mark.parametrize("N", [1, 17, 18, 19, 23, 24, 25, 28, 29, 301])
 def test_product_on_ragged_rows(neq, N):
     start, cols = graph(N, 10 * N + neq)
     rng = np.random.default_rng(N)
@@ -65,6 +65,28 @@ def test_product_on_ragged_rows(neq, N):
     ctx.close()
 
 
+@pytest.mark.parametrize("neq", [2, 3])
+@pytest.mark.parametrize("N", [85, 86, 128, 129, 300])
+def test_short_rows_fill_the_workgroups(neq, N):
+    """Rows of one or two blocks: a workgroup takes one per thread (85 or 128), the last one what is left."""
+    print("neq", neq, "N", N, flush=True)
+    two = np.arange(N) % 3 == 1
+    start = np.concatenate([[0], np.cumsum(1 + two)]).astype(np.uint32)
+    cols = np.concatenate([[i - 1, i] if two[i] else [i] for i in range(N)]).astype(np.uint32)
+    rng = np.random.default_rng(N)
+    ctx = cabi.Context(0)
+    s = cabi.System(ctx, neq=neq, graph=(start, cols, N))
+    s.reset(0.25)
+    x = rng.integers(-8, 9, N * neq).astype(np.float64)          # the sums are exact
+    b = x.reshape(N, neq).sum(1) * 0.25
+    y = np.repeat(b + np.where(two, np.roll(b, 1), 0.0), neq)
+    s.set_vector(cabi.SOLUTION, x)
+    s.apply_device(1.0, s.vector_ptr(cabi.SOLUTION), 0.0, s.vector_ptr(cabi.RHS))
+    assert np.array_equal(s.vector(cabi.RHS), y)
+    s.close()
+    ctx.close()
+
+
 @pytest.mark.parametrize("neq", [1, 2, 3])
 def test_products_are_fused(neq):
     """Row sums are fused multiply-adds in ascending order: with a a = 1 + 2 e + e^2, whose last term the rounded
@@ -101,8 +123,9 @@ def test_products_are_fused(neq):
 
 
 def test_product_of_more_rows_than_workgroups():
-    """Diagonal blocks in more rows than 2^32 work-items serve: the last rows are multiplied too."""
-    N = 2 ** 28 + 3
+    """More rows than one launch reaches (2^22 workgroups of 128 rows of one block): the last ones are multiplied
+    too."""
+    N = 2 ** 29 + 3
     ctx = cabi.Context(0)
     s = cabi.System(ctx, neq=2, graph=(np.arange(N + 1, dtype=np.uint32), np.arange(N, dtype=np.uint32), N))
     s.reset(0.5)
@@ -111,7 +134,7 @@ def test_product_of_more_rows_than_workgroups():
     print("system made", flush=True)
     s.apply_device(2.0, s.vector_ptr(cabi.SOLUTION), 1.0, s.vector_ptr(cabi.RHS))
     value = C.c_double()
-    for row in (0, 2 ** 22 * 18 - 1, 2 ** 22 * 18, N // 2, N - 2, N - 1):   # 18 rows a workgroup
+    for row in (0, N // 2, N - 5, N - 4, N - 3, N - 2, N - 1):
         for eq in (0, 1):
             cabi.check(cabi.lib().cf3hip_vector_get_value(s.h, cabi.RHS, row, eq, C.byref(value)))
             assert value.value == 2.0 * (0.5 * 3.0 + 0.5 * 3.0) + 1.0, (row, eq)
