@@ -49,7 +49,7 @@ struct SpecP1 {
   R ua[D];          // mean advection velocity u_avg
   R na[D];          // normal of the row node a
   R Q[D];           // velocity-row coefficient: skew-symmetric advection + stress diffusion + bulk
-  R tsdV, nudV, visc, m0;   // element: tau / (D^2 V), nu / (D^2 V), nu / (3 D^2 V) + tau_bulk / (D^2 V), V / (12|20)
+  R tsdV, nudV, visc, m0dt;   // element: tau / (D^2 V), nu / (D^2 V), nu / (3 D^2 V) + tau_bulk / (D^2 V), V / (12|20 dt)
   R tsu;
   R cc, cpres, pn, pp, tdo, tdd, tpc;
   int a;
@@ -201,7 +201,7 @@ struct SpecP1 {
     tsdV = tsu * rdV;
     nudV = nu * rdV;
     visc = nudV * R(1.0 / 3.0) + tbu * rdV;
-    m0 = V * R(D == 2 ? 1.0 / 12.0 : 1.0 / 20.0);
+    m0dt = (R)g.invdt * (V * R(D == 2 ? 1.0 / 12.0 : 1.0 / 20.0));
   }
 
   // coefficients of the row of local node a_
@@ -236,8 +236,8 @@ struct SpecP1 {
     pn = R(0.5) * tsdV * ni_ut + c0;   // tau_ps = tau_su
     pp = tsdV * inv_rho;
     const R invdt = (R)g.invdt;
-    tdo = invdt * (m0 + time_ii);
-    tdd = invdt * (R(2) * m0 + time_ii);
+    tdo = m0dt + invdt * time_ii;
+    tdd = tdo + m0dt;
     tpc = invdt * tsu * c0;
   }
 
@@ -863,7 +863,7 @@ __device__ __forceinline__ void assemble_lists_wg(const AsmArgs& g, const PackAr
     rec[Y::ELEM + 2] = op.visc;
     rec[Y::ELEM + 3] = op.ua[0];
     rec[Y::ELEM + 4] = op.ua[1];
-    rec[Y::ELEM + 5] = (R)g.invdt * op.m0;
+    rec[Y::ELEM + 5] = op.m0dt;
   }
   if(t < (uint32_t)Y::WORDS) s_rec[ne * Y::STRIDE + t] = R(0);   // the record of the unused list entries
   // block of this thread's list; row of the LDS rows: the first list of a block at its block, the others
