@@ -409,7 +409,7 @@ __global__ __launch_bounds__(kRT) void k_fb_x(uint64_t n, double* __restrict__ S
 // products: the product kernel forms the entries of D^-1 p (D^-1 s) it needs from r, p, v and D^-1 as it
 // gathers them, every entry by the arithmetic of k_fb_p (k_fb_s), and the row's owner stores p.  What a
 // gather reads no workgroup of the launch writes: p and v alternate between two buffers by iteration parity.
-// k_fb_x's work then starts from r, v and p.  fused_gather_blocks says where the extra gathers stop paying.
+// k_fb_x's work then starts from r, v and p.  fused_gather_rows says where the extra gathers stop paying.
 //   STAGE 1: p' = r + beta (p - omega v), y = A D^-1 p', partials rh . y
 //   STAGE 2: s = r - alpha v,             y = A D^-1 s,  partials s . s, y . s, y . y
 template<typename VR, int NEQ, int STAGE>
@@ -432,15 +432,12 @@ __global__ __launch_bounds__(kRT) void k_fb_product(uint32_t N, const uint32_t* 
   const uint32_t l = threadIdx.x & (LANES - 1);
   const uint32_t sub = WIDE ? l >> 3 : l, c0 = WIDE ? 2 * (l & 1) : 0, a0 = WIDE ? (l & 7) >> 1 : 0;
   const bool own = WIDE ? (l < 8 && (l & 1) == 0) : l == 0;
-  const uint32_t step = gridDim.x * (kRT / LANES);
-  uint32_t row = blockIdx.x * (kRT / LANES) + threadIdx.x / LANES;
+  const uint32_t row = blockIdx.x * (kRT / LANES) + threadIdx.x / LANES;
 
   uint32_t q = 0, q1 = 0;
   double m[T][RW][CW], gr[T][CW], gp[T][CW], gv[T][CW], gd[T][CW];
   double wr[RW], wp[RW], wv[RW], wh[RW];           // the owner's entries of its row
-  auto row_begin = [&] {
-    q = q1 = 0;
-    if(row >= N) return;
+  if(row < N) {
     q = row_ptr[row] + sub;
     q1 = row_ptr[row + 1];
     if(own)
@@ -451,7 +448,7 @@ __global__ __launch_bounds__(kRT) void k_fb_product(uint32_t N, const uint32_t* 
         wv[i] = v[o];
         if constexpr(STAGE == 1) { wp[i] = p[o]; wh[i] = rh[o]; }
       }
-  };
+  }
   auto load = [&] {
 #pragma unroll
     for(int k = 0; k < T; ++k) {
@@ -471,7 +468,6 @@ __global__ __launch_bounds__(kRT) void k_fb_product(uint32_t N, const uint32_t* 
       }
     }
   };
-  row_begin();
   if(q < q1) load();
 
   // the scalars of the iteration, as in k_fb_p and k_fb_s
@@ -517,7 +513,7 @@ __global__ __launch_bounds__(kRT) void k_fb_product(uint32_t N, const uint32_t* 
   double acc[ND];
 #pragma unroll
   for(int d = 0; d < ND; ++d) acc[d] = 0.;
-  while(row < N) {
+  if(row < N) {
     double ys[RW];
 #pragma unroll
     for(int i = 0; i < RW; ++i) ys[i] = 0.;
@@ -564,9 +560,6 @@ __global__ __launch_bounds__(kRT) void k_fb_product(uint32_t N, const uint32_t* 
           acc[ND > 2 ? 2 : 0] += ys[i] * ys[i];
         }
       }
-    row += step;
-    row_begin();
-    if(q < q1) load();
   }
   block_reduce_store<ND>(acc, out, gridDim.x);
 }
@@ -736,13 +729,16 @@ __global__ void k_reseed(double* S, double maxr)
 
 constexpr int kFirstBatch = 4;
 constexpr int kMaxBatch = 16;   // iterations enqueued between two host reads of the scalars
-// partials of the fused iteration: (||r||^2, rh . r), rh . v, ||s||^2, (t . s, t . t)
+// partials of the fused iteration: (||r||^2, rh . r), rh . v, ||s||^2, (t . s, t . t) or (s . s, t . s, t . t)
 constexpr size_t kFusedPartials = 2 * kMaxRedBlocks + kFusedSpmvBlocks + kMaxRedBlocks + 3 * kFusedSpmvBlocks;
-// Node blocks up to which an iteration takes three launches, by equations per node.  Measured per iteration, five
-// -> three launches (us): 4 equations 16^3 cells 30 -> 24, 24^3 (218 k blocks) 34 -> 33, 28^3 43 -> 51; 1 equation
-// (a semi-implicit step, ms) 128^2 17.2 -> 11.7, 200^2 (360 k) 25.8 -> 25.0, 256^2 39.6 -> 40.0; 3 equations
-// 64^2 (29 k) 21.3 -> 19.8, 128^2 25 -> 35.  2 equations: between their neighbours.
-inline uint64_t fused_gather_blocks(int neq) { return neq == 1 ? 360000 : neq == 2 ? 120000 : neq == 3 ? 40000 : 220000; }
+// Block rows up to which an iteration takes three launches, by equations per node (and 27 blocks for each: longer rows
+// are not measured).  The line lies at the same number of rows for rows of 7, 9, 15 and 27 blocks, FP64 and FP32 values.  Time per iteration, three launches over five: 1 equation
+// 0.78 at 13 k rows, 0.93 at 40 k, 1.03 at 55 k; 2 equations 0.83 at 8 k, 0.95 at 15 k, 1.04 at 18 k; 3 equations 0.86 at
+// 8 k, 1.04 at 10 k, 1.15 at 15 k; 4 equations 0.87 at 6.5 k, 0.93 (FP32 values 0.98) at 10 k, 0.98 (1.04) at 13 k, 1.2 at 18 k.
+// (9-block rows of 4 k: 22.9 -> 17.5, 22.9 -> 17.6, 23.5 -> 17.5, 24.4 -> 19.2 us.)
+constexpr uint32_t fused_gather_rows(int neq) { return neq == 1 ? 45000 : neq == 2 ? 16000 : neq == 3 ? 9000 : 11000; }
+// the products of such a system give every row its lanes
+static_assert(fused_gather_rows(1) <= kFusedSpmvBlocks * (kRT / 8) && fused_gather_rows(2) <= kFusedSpmvBlocks * (kRT / 16));
 
 template<typename Src, typename Dst>
 __global__ void k_convert_scaled(uint64_t n, const Src* __restrict__ a, Dst* __restrict__ b, double scale)
@@ -812,7 +808,8 @@ struct Recurrence {
     // rows per workgroup of the fused products: 16 lanes per node row, 8 for scalar rows (k_spmvn_dot)
     Gs = std::min<unsigned>(kFusedSpmvBlocks, grid_for(L.n_nodes, kRT / (L.neq == 1 ? 8 : 16)));
     part = c.red_partials.as<double>();
-    gather = fused && sizeof(R) == sizeof(double) && L.n_blocks <= fused_gather_blocks(L.neq);
+    gather = fused && sizeof(R) == sizeof(double) && L.n_nodes <= fused_gather_rows(L.neq) &&
+             L.n_blocks <= 27ull * fused_gather_rows(L.neq);
     if(fused) {
       if(!c.fused_partials.ptr) c.fused_partials.alloc(&c, sizeof(double) * kFusedPartials);
       px = c.fused_partials.as<double>();
@@ -1422,8 +1419,9 @@ void reliable_core(Lss& L, Resid resid, const cf3hip_solver_params& prm, cf3hip_
   int stall = 0;
   bool switched = false;
   // Iterations enqueued before a host read: a segment between replacements is about as long as the one
-  // before it, and launches past its stop return at once (about 5 us an iteration, a host read 12), so the
-  // first batch of a segment has the length of the last one, the next ones a few iterations
+  // before it, and launches past its stop end early (an iteration of them takes 8 us where its vectors are
+  // small and up to 40 where the loads ahead of the flag's test do not fit into the caches, 64^3 nodes and
+  // more; a host read takes 12), so the first batch of a segment has the length of the last one, the next ones a few iterations
   constexpr int kExtraBatch = 3;
   int it = 0, last = 0, batch = kFirstBatch, segment = 0;
   Scalars sc;

@@ -1,9 +1,12 @@
-"""The three-launch BiCGStab iteration of small systems on either side of its size limits, 1 to 4 equations per
-node: rows of 1 to 40 blocks, a graph whose rows are no multiple of a workgroup's, odd and even iteration counts at
-the stops, in FP64 and in the precision form on stored FP32 values (residual replacements at any parity).
+"""The three-launch BiCGStab iteration of small systems, 1 to 4 equations per node: rows of 1 to 13 blocks, graphs
+whose rows are no multiple of a workgroup's, odd and even iteration counts at the stops, in FP64 and in the
+precision form on stored FP32 values (residual replacements at any parity); and couplings in all rows on either
+side of the limits in block rows.
 
 Bars: converged, and the true residual on the matrix read back meets the tolerance to within the drift of the
 recursive residual (a factor 10, as in the other solver tests)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -12,8 +15,7 @@ from coolfluid3_amd import cabi
 pytestmark = pytest.mark.gpu
 
 
-# one row, a few rows, rows just above a workgroup's 16 or 32, and about 40 k / 130 k blocks (beyond the limit of
-# 3 and 2 equations per node, below that of 1 and 4)
+# one row, a few rows, rows just above a workgroup's 16 or 32, and thousands (20000: the five-launch form)
 @pytest.mark.parametrize("neq,N", [(q, n) for q in (1, 2, 3, 4) for n in (1, 3, 33, 700, 6000)] + [(2, 20000)])
 def test_solves_across_sizes(neq, N):
     print("neq", neq, "N", N, flush=True)
@@ -54,6 +56,40 @@ def test_solves_across_sizes(neq, N):
         s.reset_vector(cabi.SOLUTION)
         st = s.solve(cabi.solver_params(tol=tol, max_iter=500, precision=cabi.FP32))
         assert st.converged and residual(s.vector(cabi.SOLUTION)) <= 10 * tol
+    s.close()
+    ctx.close()
+
+
+# block rows up to which an iteration takes three launches
+@pytest.mark.parametrize("neq,limit", [(1, 45000), (2, 16000), (3, 9000), (4, 11000)])
+@pytest.mark.parametrize("above", [0, 1])
+def test_either_side_of_the_limits(neq, limit, above):
+    """Rows of 3 to 5 blocks with couplings everywhere and a diagonal that varies, at the limit and one row above."""
+    N = limit + above
+    print("neq", neq, "N", N, flush=True)
+    rng = np.random.default_rng(neq)
+    far = 137
+    rows = [[j for j in (i - far, i - 1, i, i + 1, i + far) if 0 <= j < N] for i in range(N)]
+    start = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.uint32)
+    ctx = cabi.Context(0)
+    s = cabi.System(ctx, neq=neq, graph=(start, np.concatenate(rows).astype(np.uint32), N))
+    s.enable_fp32()
+    s.reset(-0.12 / neq)
+    diag = rng.uniform(0.7, 2.0, N * neq)
+    cabi.check(cabi.lib().cf3hip_matrix_set_diagonal(s.h, diag.ctypes.data_as(C.c_void_p)))
+    b = rng.uniform(-1, 1, N * neq)
+    s.set_vector(cabi.RHS, b)
+    s.round_fp32()
+    rp, ci, v = s.debug_data()
+    r64 = np.repeat(np.arange(N * neq), np.diff(rp.astype(np.int64)))
+    assert np.array_equal(v[(r64 == ci)], diag)
+    for prec in (cabi.FP64, cabi.FP32):
+        for tol in (1e-4, 1e-11):
+            s.reset_vector(cabi.SOLUTION)
+            st = s.solve(cabi.solver_params(tol=tol, max_iter=500, precision=prec))
+            x = s.vector(cabi.SOLUTION)
+            res = np.linalg.norm(b - np.bincount(r64, v * x[ci], N * neq)) / np.linalg.norm(b)
+            assert st.converged and st.iterations > 2 and res <= 10 * tol, (prec, tol, st.iterations, res)
     s.close()
     ctx.close()
 
