@@ -724,8 +724,8 @@ __global__ __launch_bounds__(kThreads, sizeof(R) == sizeof(float) ? 5 : 1) void 
 // The staged reduction (assemble_wg) instead computes an element once per owned row, forms every element
 // block of 16 values, writes it to LDS and reads it back, K passes with two barriers each, and repeats the
 // combine and the rhs product for every one.
-// Measured (kernel, us, staged reduction -> block lists): FP64 tetrahedra 61^3 cells 389 -> 264, 128^3
-// 3147 -> 2179; FP32 208 -> 143, 1811 -> 1139; triangles 700^2 140 -> 120 (FP64), 81 -> 68 (FP32).
+// Measured (us, staged reduction -> block lists): FP64 tetrahedra 61^3 cells 361 -> 254, 100^3 1535 -> 1080, 128^3 (kernel
+// alone) 3147 -> 2189; FP32 215 -> 142, 920 -> 641, 1811 -> 1171; triangles 500^2 63 -> 59 (FP64), 41 -> 36 (FP32).
 // At 61^3: 1206 -> 990 VALU instructions per wave and 5/6 of the waves, 25 % fewer LDS instructions; VALU and
 // LDS are each busy about 60 % of the time with 5 to 6 workgroups per CU, and neither HBM (1.9 TB/s) nor the
 // load chain at the start bounds it: a persistent form that loads the next plan and its nodes during the block

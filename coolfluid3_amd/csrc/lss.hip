@@ -121,8 +121,9 @@ __global__ void k_spmv_mixed_generic(uint32_t N, int neq, const uint32_t* __rest
 // order: bit for bit the sums of k_spmv_generic.  A range of more than stream_blocks blocks is taken in pieces.
 // Bound by the value stream where enough workgroups fit into LDS (12 to 16 KB each, rounded to what measured best):
 // 512 x 512 quadrilaterals, neq = 3, 180 MB, one thread per scalar row 75 us (FP32 58), 256 blocks 51, 216 46.7,
-// 162 39.3 (4.9 TB/s), 128 42.1; FP32 128 37.7, 256 32.0.  4 M blocks of neq = 2 in rows of 9: 70 us (64), 162 blocks 41.8,
-// 256 33.1, 288 35.8; FP32 256 29.4, 512 26.6.
+// 162 39.3, 128 42.1; FP32 128 37.7, 256 32.0 (repeated products, values in the last-level cache; from HBM 52 us, and 900 x
+// 900, 565 MB, 296 -> 161 us, 3.5 TB/s).  4 M blocks of neq = 2 in rows of 9: 70 us (64), 162 blocks 41.8, 256 33.1, 288 35.8;
+// FP32 256 29.4, 512 26.6.
 template<typename T>
 constexpr int stream_blocks(int neq) { return sizeof(T) == 8 ? (neq == 2 ? 256 : 162) : (neq == 2 ? 512 : 256); }
 // Rows of a workgroup: as many as fill stream_blocks on average, at most one thread per scalar row.  4 M blocks in rows
