@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <cstdlib>
 #include <memory>
 #include <string>
 #include <type_traits>
@@ -168,7 +169,8 @@ struct Lss {
   // Dirichlet conditions applied since the last reset (needed by the matrix-free FP64 residual):
   // per dof the first value (column elimination) and the last value (row / solution)
   // (condition i, in order of first application: its dof, first and last value; bc_slot: condition + 1 of a dof)
-  std::vector<uint32_t> bc_slot;   // dofs entries, made by the first condition of the system
+  // dofs entries, made by the first condition of the system: zeroed pages, of which a call touches those of its dofs
+  std::unique_ptr<uint32_t[], void (*)(void*)> bc_slot{nullptr, std::free};
   std::vector<uint32_t> bc_order;
   std::vector<double> bc_first, bc_last;
   std::vector<uint64_t> bc_call;   // per condition the call that applied it last

@@ -10,6 +10,8 @@
 
 #include <cctype>
 #include <cstdio>
+#include <cstdlib>
+#include <new>
 #include <string>
 
 #include "internal.hpp"
@@ -680,13 +682,17 @@ void lss_dirichlet(Lss& L, uint32_t nbc, const uint32_t* nodes, const uint32_t* 
   // earlier one since the last reset) gets its column eliminated with that first value; every
   // condition sets the row to the identity and the rhs / solution to its value, so the last value
   // wins there (TrilinosFEVbrMatrix::symmetric_dirichlet leaves an already zero column untouched).
-  // A table over the dofs finds a dof's condition, and the lists go to the device in one copy: with hash maps,
+  // A table over the dofs finds a dof's condition (never filled as a whole: that took 5 ms on the first call at 128^3
+  // tetrahedra), and the lists go to the device in one copy: with hash maps,
   // eight buffers allocated and freed and ten copies a call took 8.0 ms for the 50 k conditions of the 64^3 cube
   // (0.5 ms now), 2.5 ms for the 17 k of a 37^3 channel (0.2).
   for(uint32_t b = 0; b < nbc; ++b)
     if(nodes[b] >= L.n_nodes || eqs[b] >= (uint32_t)neq)
       CF3_THROW(CF3HIP_ERR_INVALID_ARG, "Dirichlet condition on a dof outside the system");
-  if(L.bc_slot.empty()) L.bc_slot.assign(L.dofs, 0);
+  if(!L.bc_slot) {
+    L.bc_slot.reset(static_cast<uint32_t*>(std::calloc(L.dofs, sizeof(uint32_t))));
+    if(!L.bc_slot) throw std::bad_alloc();
+  }
   const uint64_t call = ++L.bc_calls;
   const uint32_t before = (uint32_t)L.bc_order.size();   // conditions from here on are fresh
   std::vector<uint32_t> here;                            // conditions of this call in first-appearance order
