@@ -727,8 +727,14 @@ __global__ void k_reseed(double* S, double maxr)
   S[S_SCONV] = 0.; S[S_STOP] = 0.; S[S_MAXR] = maxr; S[S_MAXR_ODD] = maxr;
 }
 
+// Iterations enqueued between two host reads of the scalars, after `done` of them: as many again, 4 to 16.  A read costs
+// 40 to 80 us of idle device, an iteration enqueued past the stop 8 to 40.  Solves of 1, 3, 5, 7 iterations, us, batches of
+// 1, 2, 4 ... / 4, 8, 16 / this: 262144 rows of 9 blocks, 1 equation, 187, 312, 456, 552 / 231, 301, 514, 583 / 230, 299, 456, 523;
+// 270000 of 15 blocks, 4 equations, 635, 1223, 1836, 2379 / 678, 1156, 1886, 2359 / 678, 1150, 1763, 2241; 4096 of 9 blocks, 2
+// equations, 120, 199, 288, 296 / 147, 149, 277, 278 / 141, 143, 234, 236.
 constexpr int kFirstBatch = 4;
-constexpr int kMaxBatch = 16;   // iterations enqueued between two host reads of the scalars
+constexpr int kMaxBatch = 16;
+inline int next_batch(int done) { return std::min(std::max(done, kFirstBatch), kMaxBatch); }
 // partials of the fused iteration: (||r||^2, rh . r), rh . v, ||s||^2, (t . s, t . t) or (s . s, t . s, t . t)
 constexpr size_t kFusedPartials = 2 * kMaxRedBlocks + kFusedSpmvBlocks + kMaxRedBlocks + 3 * kFusedSpmvBlocks;
 // Block rows up to which an iteration takes three launches, by equations per node (and 27 blocks for each: longer rows
@@ -995,7 +1001,7 @@ int bicgstab(Lss& L, const R* b, R* x, R* work, double tol, int maxit, bool& con
       conv = sc.v[S_SCONV] != 0. || sc.v[S_RN2] <= thr2;
       break;
     }
-    batch = std::min(2 * batch, kMaxBatch);
+    batch = next_batch(it);
   }
   spmvs = 1 + 2 * it;
   return it;
@@ -1430,7 +1436,7 @@ void reliable_core(Lss& L, Resid resid, const cf3hip_solver_params& prm, cf3hip_
     read_scalars(c, sc);
     it = (int)sc.v[S_ITER];
     if(sc.v[S_STOP] == 0.) {
-      batch = segment == 0 ? std::min(2 * batch, kMaxBatch) : kExtraBatch;
+      batch = segment == 0 ? next_batch(it) : kExtraBatch;
       continue;
     }
     // reliable update: move the increment into the FP64 solution, replace the residual
