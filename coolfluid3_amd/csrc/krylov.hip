@@ -1436,7 +1436,7 @@ void reliable_core(Lss& L, Resid resid, const cf3hip_solver_params& prm, cf3hip_
     read_scalars(c, sc);
     it = (int)sc.v[S_ITER];
     if(sc.v[S_STOP] == 0.) {
-      batch = segment == 0 ? next_batch(it) : kExtraBatch;
+      batch = segment == 0 ? std::min(2 * batch, kMaxBatch) : kExtraBatch;
       continue;
     }
     // reliable update: move the increment into the FP64 solution, replace the residual
